@@ -387,11 +387,14 @@ void BipartiteGraphAnnealer<real>::computeFields(int side) {
             fieldRefreshF32MFMA(f.ptr, f.n, Qin, nOutP, K, m_, NwIn, ldE, (float *)d_dE_.ptr, dev_->stream());
         }
     } else {
-        /* vector form: dE[y][o] = sum_{k < nIn} q[y][k] B[k][o] with B = J^T (side 1) or J (side 0) */
+        /* dE[y][o] = sum_{k < nIn} q[y][k] B[k][o] with B = J^T (side 1) or J (side 0) */
         const real *B = side ? d_JT_.ptr : d_J_.ptr;
-        fieldRefresh<real>(B, nIn, nOutP, nOutP, Qin, m_, NwIn, ldE, d_dE_.ptr, dev_->stream());
+        if (sizeof(real) == 8 && !refreshVector_)
+            fieldRefreshF64MFMA((const double *)B, nIn, roundUp(nOut, 16), nOutP, Qin, m_, NwIn, ldE,
+                                (double *)d_dE_.ptr, dev_->stream());
+        else
+            fieldRefresh<real>(B, nIn, nOutP, nOutP, Qin, m_, NwIn, ldE, d_dE_.ptr, dev_->stream());
     }
-    (void)nOut;
 }
 
 template <class real>

@@ -707,9 +707,9 @@ void DenseGraphAnnealer<real>::refreshFields(bool always) {
         fieldsDirty_ = false;
         return;
     }
-    /* F = Q . J in the field format: MFMA for float solvers, vector FMA for
-     * double (and on request, as the cross-check of the MFMA kernels) */
-    const bool mfma = sizeof(real) == 4 && !refreshVector_;
+    /* F = Q . J in the field format on the matrix units (on request by the
+     * vector kernel, their cross-check) */
+    const bool mfma = !refreshVector_;
     if (mfma)
         ensureFragments();
     if (fieldFormat_ == fieldFP8) {
@@ -727,6 +727,9 @@ void DenseGraphAnnealer<real>::refreshFields(bool always) {
                                dev_->stream());
         else
             fieldRefresh<float>(d_Jsplit_.ptr, N_, Np_, Np_, d_Q_.ptr, m_, Nw_, Np_, (float *)d_F_.ptr, dev_->stream());
+    } else if (mfma && sizeof(real) == 8) {
+        fieldRefreshF64MFMA((const double *)d_J_.ptr, N_, Np_, Np_, d_Q_.ptr, m_, Nw_, Np_, (double *)d_F_.ptr,
+                            dev_->stream());
     } else if (mfma) {
         fieldRefreshF32MFMA(d_frag32_.ptr, d_frag32_.n, d_Q_.ptr, Np_, Np_, m_, Nw_, Np_, (float *)d_F_.ptr,
                             dev_->stream());

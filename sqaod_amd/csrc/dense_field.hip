@@ -5,9 +5,9 @@
  * annealer recomputes the same J-row . q-row dot per attempt,
  * CPUDenseGraphAnnealer.cpp:257) and the bipartite half-steps' dEmat.
  *
- * This file holds the vector-ALU form (fp64 J for double solvers, and fp32 J
- * as the cross-check the MFMA kernels of dense_field_mfma.hip are tested
- * against), the bf16 hi+lo split of J and the FP8 (e4m3) quantization of J.
+ * This file holds the vector-ALU form (the cross-check the MFMA kernels of
+ * dense_field_mfma.hip are tested against), the bf16 hi+lo split of J and the
+ * FP8 (e4m3) quantization of J.
  * Each block owns 256 columns and a tile of slices; spins enter as sign flips
  * of J, so the products are exact.
  */

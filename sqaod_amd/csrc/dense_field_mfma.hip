@@ -14,6 +14,8 @@
  *  - fp8:    J as e4m3 bytes with a power-of-two scale per column, spins
  *    +-1 exact in e4m3, v_mfma_scale_f32_16x16x128_f8f6f4 with unit block
  *    scales; the column scale multiplies the reduced sum (exactly).
+ *  - fp64:   J as it is stored, v_mfma_f64_16x16x4_f64 (a kernel of its own,
+ *    fieldRefreshF64Kernel).
  *
  * J is read from a copy laid out in MFMA fragment order, built once per
  * problem: for column block cb (16 columns) and k-block kb, the 64 lanes'
@@ -262,6 +264,102 @@ __global__ __launch_bounds__(kBlockThreads) void fieldRefreshBF16x3Kernel(const 
     refreshBF16Block<3>(frag, Qbits, K, m, Nw, ldF, F, blockIdx.x, red, lut);
 }
 
+
+/* Double solvers: F[y][c] = sum_{k < K} q[y][k] B[k][c] with B row-major, as it
+ * is stored (the dense annealer's J, the bipartite one's J or J^T).
+ *
+ * A block of 4 waves owns 16 columns and RT 16-row tiles; wave w takes the
+ * k-blocks of 32 (one spin word a row) w, w + 4, ..., eight
+ * v_mfma_f64_16x16x4_f64 per tile each, and the four partial tiles are added
+ * in LDS in the order ((P0 + P1) + P2) + P3.  Lane L supplies B[k][c] and the
+ * spin of row L % 16 for k = 32 kb + 4 t + L / 16: a load instruction reads
+ * four 128-byte row pieces, and the next k-block's loads are in flight while
+ * this one's products run.
+ *
+ * A matrix instruction takes 64 cycles, so the product itself is short (under
+ * 2 us at N=500, m=125); at these sizes the kernel is bound by filling the
+ * chip and by one memory round trip per k-block.  Hence a column block of 16,
+ * the k-range over the four SIMDs of a CU, and RT = 1 until every CU has two
+ * blocks: the vector kernel this replaced keeps 256 columns and 32 rows a
+ * block, 8 blocks at that size.  Measured: 6.0 us against the vector kernel's
+ * 245.6 us at N=500, m=125; 4.6 against 124.4 us for the bipartite half-steps
+ * at 200 + 301 spins, m=125.
+ */
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+constexpr int kF64KBlock = 32;
+constexpr int kF64Steps = kF64KBlock / 4;
+
+template <int RT>
+__global__ __launch_bounds__(kBlockThreads) void fieldRefreshF64Kernel(const double *B, int K, int ldB,
+                                                                       const uint32_t *Qbits, int m, int Nw, int ldF,
+                                                                       double *F) {
+    __shared__ double red[kSplitK][RT * 4][kWave];
+    const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+    const int c = lane & 15, g = lane >> 4;
+    const int y0 = blockIdx.y * 16 * RT;
+    const double *Bc = B + blockIdx.x * 16 + c;
+    const int nK = (K + kF64KBlock - 1) / kF64KBlock; /* nK <= Nw: K <= 32 Nw */
+    f64x4 acc[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+        acc[t] = f64x4{0., 0., 0., 0.};
+    double b[2][kF64Steps];
+    uint32_t qw[2][RT];
+    /* rows of B past K and slices past m are read at the last valid one; the
+     * former enter as zeros, the latter's sums are not stored */
+    auto fetch = [&](int buf, int kb) {
+#pragma unroll
+        for (int t = 0; t < kF64Steps; ++t) {
+            const int k = kb * kF64KBlock + 4 * t + g;
+            const double v = Bc[(size_t)(k < K ? k : K - 1) * ldB];
+            b[buf][t] = k < K ? v : 0.;
+        }
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            const int y = y0 + 16 * r + c;
+            qw[buf][r] = Qbits[(size_t)(y < m ? y : m - 1) * Nw + kb];
+        }
+    };
+    auto compute = [&](int buf) {
+#pragma unroll
+        for (int t = 0; t < kF64Steps; ++t)
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+                const double q = ((qw[buf][r] >> (4 * t + g)) & 1u) ? 1. : -1.;
+                acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(q, b[buf][t], acc[r], 0, 0, 0);
+            }
+    };
+    if (w < nK)
+        fetch(0, w);
+    for (int kb = w; kb < nK; kb += 2 * kSplitK) {
+        if (kb + kSplitK < nK)
+            fetch(1, kb + kSplitK);
+        compute(0);
+        if (kb + kSplitK >= nK)
+            break;
+        if (kb + 2 * kSplitK < nK)
+            fetch(0, kb + 2 * kSplitK);
+        compute(1);
+    }
+    /* register r of lane L: row 4 r + L / 16, column L % 16 of the tile */
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            red[w][4 * t + r][lane] = acc[t][r];
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        /* thread (w, lane) adds row piece r = w of each tile */
+        const int y = y0 + 16 * t + 4 * w + g;
+        double s = red[0][4 * t + w][lane];
+#pragma unroll
+        for (int p = 1; p < kSplitK; ++p)
+            s += red[p][4 * t + w][lane];
+        if (y < m)
+            F[(size_t)y * ldF + blockIdx.x * 16 + c] = s;
+    }
+}
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 constexpr int kDepth8 = 2; /* fp8: k-blocks of 128 per super-block (256 k = 8 spin words) */
@@ -595,6 +693,21 @@ void fieldRefreshF32MFMA(const uint16_t *d_frag, size_t fragElems, const uint32_
     SQ_THROW_IF(fragElems < fieldFragElemsF32(nCols, K), "fp32 fragment buffer too small");
     fieldRefreshBF16x3Kernel<<<nCols / 16, kBlockThreads, 0, stream>>>(reinterpret_cast<const uint4 *>(d_frag),
                                                                        d_Qbits, K, m, Nw, ldF, d_F);
+    HIP_CHECK(hipGetLastError());
+}
+
+void fieldRefreshF64MFMA(const double *d_B, int K, int nCols, int ldB, const uint32_t *d_Qbits, int m, int Nw,
+                         int ldF, double *d_F, hipStream_t stream) {
+    SQ_THROW_IF(nCols <= 0 || nCols % 16 != 0, "field GEMM: %d output columns is not a positive multiple of 16",
+                nCols);
+    SQ_THROW_IF(K <= 0 || K > Nw * 32 || ldB < nCols || ldF < nCols || m <= 0, "field GEMM: inconsistent shape");
+    /* row tiles per block: as many as leave two blocks to each of 256 CUs (a
+     * tile more reads B's columns once for twice the slices) */
+    const int colBlocks = nCols / 16, rowTiles = divru(m, 16);
+    const int rt = colBlocks * divru(rowTiles, 4) >= 512 ? 4 : colBlocks * divru(rowTiles, 2) >= 512 ? 2 : 1;
+    const dim3 grid((unsigned)colBlocks, (unsigned)divru(rowTiles, rt));
+    auto *kernel = rt == 4 ? fieldRefreshF64Kernel<4> : rt == 2 ? fieldRefreshF64Kernel<2> : fieldRefreshF64Kernel<1>;
+    kernel<<<grid, kBlockThreads, 0, stream>>>(d_B, K, ldB, d_Qbits, m, Nw, ldF, d_F);
     HIP_CHECK(hipGetLastError());
 }
 

@@ -116,6 +116,12 @@ template <class real>
 void fieldRefresh(const real *d_B, int K, int nCols, int ldB, const uint32_t *d_Qbits, int m, int Nw, int ldF,
                   real *d_F, hipStream_t stream);
 
+/* The double solvers' form on the FP64 matrix units (dense_field_mfma.hip):
+ * fieldRefresh<double>'s product with the same arguments, for nCols a
+ * multiple of 16; every product exact, sums in FP64 in a fixed order. */
+void fieldRefreshF64MFMA(const double *d_B, int K, int nCols, int ldB, const uint32_t *d_Qbits, int m, int Nw,
+                         int ldF, double *d_F, hipStream_t stream);
+
 /* MFMA forms (dense_field_mfma.hip): F[y][c] = sum_k q[y][k] B[c][k] for
  * c < nCols (a multiple of 16), k < K (a multiple of 256, Nw = K/32 spin words
  * per row), fp32 accumulation, F row stride ldF.  B (rows x ld floats, zero

@@ -75,3 +75,19 @@ def test_incremental_fields_track_spins(oracle, rocm, form):
     F = an.get_fields().astype(np.float64)
     assert np.array_equal(F, host_fields(oracle, W, np.stack(an.get_q())))
     assert an.get_counters()["flips"] > 0
+
+
+@pytest.mark.parametrize("N,m", [(1, 1), (5, 3), (31, 17), (33, 16), (129, 33), (500, 125), (1000, 200), (2100, 256)])
+def test_field_gemm_fp64(oracle, rocm, N, m):
+    """The double solvers' matrix-unit fields: exact on integer problems at
+    k-blocks of 32, 16-slice tiles and one to four tiles per block, whole and
+    ragged; on N(0,1) within N ulps of sum |J| (a sum of N exact products in
+    any order is off by less than N 2^-53 sum |J|)."""
+    an = annealer(rocm, dense_int_W(N, SEED_BASE + N, dtype=np.float64), m)
+    W = dense_int_W(N, SEED_BASE + N, dtype=np.float64)
+    assert np.array_equal(an.get_fields(), host_fields(oracle, W, np.stack(an.get_q())))
+    W = dense_normal_W(N, SEED_BASE + N, dtype=np.float64)
+    an = annealer(rocm, W, m)
+    F, J = an.get_fields(), oracle.dense_hamiltonian(W)[1]
+    bound = 2.0 * N * 2.0 ** -53 * np.abs(J).sum(axis=1)  # the host product's own rounding as well
+    assert np.all(np.abs(F - host_fields(oracle, W, np.stack(an.get_q()))) <= bound)
