@@ -65,7 +65,9 @@ void Formulas<real>::run(QuadFormArgs<real> a, const real *A, size_t nA, const r
         a.lin1 = d1.ptr;
     }
     a.E = dE.ptr;
-    quadForm<real>(a, nOut, st);
+    DevBuf<unsigned char> dWork;
+    dWork.allocate(quadFormWorkBytes(a.nu, a.nv, a.nV, a.twoD != 0));
+    quadForm<real>(a, nOut, dWork.ptr, dWork.n, st);
     HIP_CHECK(hipMemcpyAsync(E, dE.ptr, (size_t)nOut * sizeof(real), hipMemcpyDeviceToHost, st));
     dev.synchronize();
 }

@@ -409,8 +409,10 @@ struct QuadFormArgs {
     int nu, nv, nV, twoD;
     real *E;
 };
+/* d_work: quadFormWorkBytes(nu, nv, nV, twoD) bytes of scratch. */
+size_t quadFormWorkBytes(int nu, int nv, int nV, bool twoD);
 template <class real>
-void quadForm(const QuadFormArgs<real> &a, int nOut, hipStream_t stream);
+void quadForm(const QuadFormArgs<real> &a, int nOut, void *d_work, size_t workBytes, hipStream_t stream);
 
 /* sum_y q_y . q_(y+1)%m (the Trotter coupling of getSystemE), in double. */
 void spinDotSum(const uint32_t *d_Qbits, int N, int m, int Nw, double *d_out, hipStream_t stream);

@@ -131,3 +131,39 @@ def test_shape_errors(F):
     with pytest.raises(RuntimeError):
         F.bipartite_graph_batch_calculate_E(np.ones(3), np.ones(2), np.ones((3, 3)), np.zeros((1, 3), np.int8),
                                             np.zeros((1, 2), np.int8), np.float32)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,B", [(64, 5), (65, 1), (65, 33), (96, 32), (97, 64), (300, 31), (1001, 70)])
+def test_dense_batch_energy_tiles(F, dtype, N, B):
+    """Both sides of the size from which the energies are formed on the matrix
+    units (65 x 65), whole and ragged tiles of 32: exact on integers, and an
+    infinite weight counts only where both its bits are set."""
+    rng = np.random.default_rng(SEED_BASE + N)
+    W, X = int_sym(N, SEED_BASE + N), rng.integers(0, 2, (B, N)).astype(np.int8)
+    exact = np.sum((X @ W) * X, axis=1)
+    assert np.array_equal(F.dense_graph_batch_calculate_E(W, X, dtype), exact.astype(dtype))
+    W[3, N - 1] = W[N - 1, 3] = np.inf
+    both = (X[:, 3] & X[:, N - 1]).astype(bool)
+    E = F.dense_graph_batch_calculate_E(W, X, dtype)
+    assert np.all(np.isposinf(E[both])) and np.array_equal(E[~both], exact[~both].astype(dtype))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N0,N1,B0,B1", [(65, 64, 3, 40), (200, 33, 33, 1), (31, 500, 64, 65)])
+def test_bipartite_energy_tiles(F, dtype, N0, N1, B0, B1):
+    """All pairs and pairwise, ragged in each dimension, and an infinite b1
+    that counts only where its bit is set."""
+    rng = np.random.default_rng(SEED_BASE + N0 + N1)
+    b0, b1 = rng.integers(-4, 5, N0).astype(np.float64), rng.integers(-4, 5, N1).astype(np.float64)
+    W = rng.integers(-4, 5, (N1, N0)).astype(np.float64)
+    x0, x1 = rng.integers(0, 2, (B0, N0)).astype(np.int8), rng.integers(0, 2, (B1, N1)).astype(np.int8)
+    exact = x1 @ W @ x0.T + (x0 @ b0)[None, :] + (x1 @ b1)[:, None]
+    assert np.array_equal(F.bipartite_graph_batch_calculate_E_2d(b0, b1, W, x0, x1, dtype), exact.astype(dtype))
+    n = min(B0, B1)
+    assert np.array_equal(F.bipartite_graph_batch_calculate_E(b0, b1, W, x0[:n], x1[:n], dtype),
+                          np.diag(exact[:n, :n]).astype(dtype))
+    b1[2] = np.inf
+    E = F.bipartite_graph_batch_calculate_E_2d(b0, b1, W, x0, x1, dtype)
+    on = x1[:, 2].astype(bool)
+    assert np.all(np.isposinf(E[on])) and np.array_equal(E[~on], exact[~on].astype(dtype))
