@@ -4,15 +4,15 @@
  * harnesses that forbid hipMalloc).  It runs the scan of dense_bf.hip -- the
  * same kernels and the same list rule as DenseGraphBFSearcher::search -- but
  * the problem and the results are the caller's device buffers and every
- * intermediate (W in double, the low-bit energy table, the search state and
- * the per-block minima, counts and offsets) lives in `scratch`, a static
+ * intermediate (W in double, the low-bit tables, the search state and the
+ * per-unit minima, list of units and places) lives in `scratch`, a static
  * device array of this library (kScratchBytes per GPU, held until the
  * process ends).  No call allocates or frees memory.
  *
  * Every call on one GPU uses that GPU's one array: calls that overlap on a
  * GPU (two host threads, or two streams whose work overlaps) race.  Each call
- * re-initialises the state it reads (W, the table and the search state are
- * written by the set-up kernel; block entries are written by the scan before
+ * re-initialises the state it reads (W, the tables and the search state are
+ * written by the set-up kernels; unit entries are written by the scan before
  * they are read), so a call never sees the previous call's contents.
  */
 #include <cfloat>
@@ -33,19 +33,19 @@ namespace {
 constexpr int kMaxN = 63;
 constexpr unsigned long long kMaxTile = 1ull << 26;
 constexpr unsigned long long kMinSpan = 1ull << 26; /* as the searcher: one call fills the GPU */
-constexpr int kMaxBlocks = (int)(kMinSpan >> (kBFMaxLowBits + 4)) + 2;
+constexpr int kMaxUnits = 514; /* a span's: bfPlan makes at most 512, cut at both ends */
 
 /* byte offsets inside scratch, each 256-aligned */
 constexpr size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 constexpr size_t kOffW = 0;
-constexpr size_t kOffEL = align256(kOffW + sizeof(double) * kMaxN * kMaxN);
-constexpr size_t kOffState = align256(kOffEL + sizeof(double) * (1u << kBFMaxLowBits));
-constexpr size_t kOffBlockMin = align256(kOffState + 64);
-constexpr size_t kOffBlockCnt = align256(kOffBlockMin + sizeof(double) * kMaxBlocks);
-constexpr size_t kOffOffsets = align256(kOffBlockCnt + sizeof(unsigned) * kMaxBlocks);
-constexpr size_t kEnd = align256(kOffOffsets + sizeof(unsigned long long) * kMaxBlocks);
+constexpr size_t kOffTab = align256(kOffW + sizeof(double) * kMaxN * kMaxN);
+constexpr size_t kOffState = align256(kOffTab + sizeof(double) * kBFTableDoubles);
+constexpr size_t kOffUnitMin = align256(kOffState + sizeof(BFState<double>));
+constexpr size_t kOffHits = align256(kOffUnitMin + sizeof(double) * kMaxUnits);
+constexpr size_t kOffSlots = align256(kOffHits + sizeof(unsigned) * kMaxUnits);
+constexpr size_t kEnd = align256(kOffSlots + sizeof(unsigned long long) * kMaxUnits);
 static_assert(kEnd <= kScratchBytes, "scratch layout exceeds the static array");
-static_assert(sizeof(BFState<double>) <= 64, "state slot");
+static_assert(sizeof(BFState<float>) <= sizeof(BFState<double>), "state slot");
 
 std::mutex g_mu;
 unsigned char *g_addr[64] = {}; /* scratch's device address per GPU ordinal */
@@ -66,30 +66,15 @@ unsigned char *scratchOnCurrentDevice() {
     return g_addr[dev];
 }
 
-/* W (real, N x N, the caller's) -> sgn * W in double; the low-bit energy
- * table EL[xL] = sum_{b in xL} sum_{b2 in xL} W[N-1-b][N-1-b2] in the order
- * the searcher's prepare() sums it on the host (b ascending, a partial sum
- * per b); the state reset to (FLT_MAX, 0) (CPUDenseGraphBFSearcher.cpp:65). */
+/* W (real, N x N, the caller's) -> sgn * W in double; the state reset to
+ * (FLT_MAX, 0) (CPUDenseGraphBFSearcher.cpp:65). */
 template <class real>
-__global__ __launch_bounds__(256) void bfNoallocSetupKernel(const real *W, int N, double sgn, int L, double *dW,
-                                                            double *EL, BFState<real> *st) {
+__global__ __launch_bounds__(256) void bfNoallocSetupKernel(const real *W, int N, double sgn, double *dW,
+                                                            BFState<real> *st) {
     for (int i = threadIdx.x; i < N * N; i += blockDim.x)
         dW[i] = sgn * (double)W[i];
-    __syncthreads();
-    for (int xL = threadIdx.x; xL < (1 << L); xL += blockDim.x) {
-        double e = 0.;
-        for (int b = 0; b < L; ++b) {
-            if (!((xL >> b) & 1))
-                continue;
-            const double *Wr = dW + (size_t)(N - 1 - b) * N;
-            double s = 0.;
-            for (int b2 = 0; b2 < L; ++b2)
-                if ((xL >> b2) & 1)
-                    s += Wr[N - 1 - b2];
-            e += s;
-        }
-        EL[xL] = e;
-    }
+    for (int i = threadIdx.x; i < (kBFArriveGroups + 1) * kBFArriveStride; i += blockDim.x)
+        st->arrived[i] = 0;
     if (threadIdx.x == 0) {
         st->Emin = (real)FLT_MAX;
         st->count = 0;
@@ -118,21 +103,21 @@ void searchNoalloc(const real *d_W, int N, int optimize, unsigned long long tile
         cap = xMax;
     unsigned char *base = scratchOnCurrentDevice();
     double *dW = (double *)(base + kOffW);
-    double *EL = (double *)(base + kOffEL);
+    double *tab = (double *)(base + kOffTab);
     BFState<real> *st = (BFState<real> *)(base + kOffState);
-    real *blockMin = (real *)(base + kOffBlockMin);
-    unsigned *blockCnt = (unsigned *)(base + kOffBlockCnt);
-    unsigned long long *offsets = (unsigned long long *)(base + kOffOffsets);
+    real *unitMin = (real *)(base + kOffUnitMin);
+    unsigned *hits = (unsigned *)(base + kOffHits);
+    unsigned long long *slots = (unsigned long long *)(base + kOffSlots);
 
     const BFPlan plan = bfPlan(N);
     const double sgn = optimize ? -1. : 1.;
-    bfNoallocSetupKernel<real><<<1, 256, 0, stream>>>(d_W, N, sgn, plan.L, dW, EL, st);
+    bfNoallocSetupKernel<real><<<1, 256, 0, stream>>>(d_W, N, sgn, dW, st);
     HIP_CHECK(hipGetLastError());
+    bfTables(dW, plan, tab, stream);
     const unsigned long long span = cap > kMinSpan ? cap : kMinSpan;
     for (unsigned long long xb = 0; xb < xMax; xb += span) {
         const unsigned long long xe = (xMax - xb) < span ? xMax : xb + span;
-        bfSearchRange<real>(dW, EL, plan, xb, xe, st, cap, blockMin, blockCnt, offsets, kMaxBlocks, d_xList,
-                            stream);
+        bfSearchRange<real>(dW, tab, plan, xb, xe, st, cap, unitMin, hits, slots, kMaxUnits, d_xList, stream);
     }
     bfNoallocResultKernel<real><<<1, 1, 0, stream>>>(st, sgn, cap, d_Emin, d_n);
     HIP_CHECK(hipGetLastError());

@@ -21,8 +21,8 @@ namespace sqaod_rocm {
 
 namespace {
 
-/* spans scanned per searchRange call: at least 2^26 candidates (1024 blocks
- * of 65,536), so one call fills the GPU */
+/* spans scanned per searchRange call: at least 2^26 candidates (512 blocks of
+ * 131,072), so one call fills the GPU */
 constexpr unsigned long long kMinSpan = 1ull << 26;
 
 }  // namespace
@@ -100,42 +100,21 @@ void DenseGraphBFSearcher<real>::prepare() {
     }
     plan_ = bfPlan(N_);
     span_ = std::max((unsigned long long)tileSize_, kMinSpan);
-    const unsigned long long unit = 1ull << (plan_.L + plan_.lgR);
     /* a span may straddle unit boundaries at both ends */
-    maxBlocks_ = (int)(std::min(span_, xMax_) / unit + 2);
-
-    /* EL[xL] = sum_{b, b'} x_b x_b' W[N-1-b][N-1-b'], double, fixed order */
-    const int L = plan_.L, N = N_;
-    std::vector<double> EL((size_t)1 << L);
-    for (int xL = 0; xL < (1 << L); ++xL) {
-        double e = 0.;
-        for (int b = 0; b < L; ++b) {
-            if (!((xL >> b) & 1))
-                continue;
-            const double *Wr = W_.data() + (size_t)(N - 1 - b) * N;
-            double s = 0.;
-            for (int b2 = 0; b2 < L; ++b2)
-                if ((xL >> b2) & 1)
-                    s += Wr[N - 1 - b2];
-            e += s;
-        }
-        EL[xL] = e;
-    }
+    maxUnits_ = (int)((std::min(span_, xMax_) >> plan_.U) + 2);
     d_W_.allocate(W_.size());
-    d_EL_.allocate(EL.size());
+    d_tab_.allocate(kBFTableDoubles);
     d_state_.allocate(1);
-    d_blockMin_.allocate((size_t)maxBlocks_);
-    d_blockCnt_.allocate((size_t)maxBlocks_);
-    d_offsets_.allocate((size_t)maxBlocks_);
+    d_unitMin_.allocate((size_t)maxUnits_);
+    d_hits_.allocate((size_t)maxUnits_);
+    d_slots_.allocate((size_t)maxUnits_);
     d_xList_.allocate((size_t)tileSize_);
-    BFState<real> st;
+    BFState<real> st{};
     st.Emin = (real)FLT_MAX; /* CPUDenseGraphBFSearcher.cpp:65 */
-    st.count = 0;
     HIP_CHECK(hipMemcpyAsync(d_W_.ptr, W_.data(), W_.size() * sizeof(double), hipMemcpyHostToDevice, dev_->stream()));
-    HIP_CHECK(hipMemcpyAsync(d_EL_.ptr, EL.data(), EL.size() * sizeof(double), hipMemcpyHostToDevice,
-                             dev_->stream()));
     HIP_CHECK(hipMemcpyAsync(d_state_.ptr, &st, sizeof(st), hipMemcpyHostToDevice, dev_->stream()));
-    dev_->synchronize(); /* the host vectors go out of scope */
+    bfTables(d_W_.ptr, plan_, d_tab_.ptr, dev_->stream());
+    dev_->synchronize(); /* the host state goes out of scope */
     Emin_ = st.Emin;
     xList_.clear();
     E_.clear();
@@ -151,9 +130,8 @@ bool DenseGraphBFSearcher<real>::searchRange(unsigned long long *curXEnd) {
     const unsigned long long xb = x_;
     const unsigned long long xe = std::min(x_ + span_, xMax_);
     if (xb < xe)
-        bfSearchRange<real>(d_W_.ptr, d_EL_.ptr, plan_, xb, xe, d_state_.ptr, (unsigned long long)tileSize_,
-                            d_blockMin_.ptr, d_blockCnt_.ptr, d_offsets_.ptr, maxBlocks_, d_xList_.ptr,
-                            dev_->stream());
+        bfSearchRange<real>(d_W_.ptr, d_tab_.ptr, plan_, xb, xe, d_state_.ptr, (unsigned long long)tileSize_,
+                            d_unitMin_.ptr, d_hits_.ptr, d_slots_.ptr, maxUnits_, d_xList_.ptr, dev_->stream());
     x_ = xe;
     if (curXEnd)
         *curXEnd = x_;

@@ -194,32 +194,40 @@ void bipartiteFlipPhase(const BGFlipArgs<real> &a, int nSlices, hipStream_t stre
 
 /* ---------------- dense brute-force search (dense_bf.hip) ---------------- */
 
-constexpr int kBFMaxLowBits = 12;      /* low bits of x enumerated per block (2^12-entry LDS table) */
-constexpr int kBFMaxHighPatterns = 16; /* high patterns per block */
-
-/* Split of x into high and low bits for N (<= 63) */
+/* Split of x's N <= 63 bits: units of 2^U consecutive x (U = 12 + nC), nH high
+ * bits above (N < U: one unit, the bits past N - 1 do not exist) */
 struct BFPlan {
-    int N, L, nH, Llo, lgR, R;
+    int N, nC, U, nH;
 };
 BFPlan bfPlan(int N);
 
-/* Device-resident search state: the minimum so far and the list length. */
+/* Device-resident search state: the minimum so far, the list length, and what
+ * the two launches of a range hand over (`arrived`, a scan's counters of ended
+ * blocks, starts at 0). */
+constexpr int kBFArriveGroups = 16, kBFArriveStride = 32; /* 128 bytes apart */
 template <class real>
 struct BFState {
     real Emin;
-    unsigned long long count;
+    unsigned long long count, base;
+    unsigned nHit, ticket;
+    unsigned arrived[(kBFArriveGroups + 1) * kBFArriveStride];
 };
 
-/* Scans x in [xb, xe) (E = x^T W x with W: N x N double, EL: the 2^L-entry
- * low-bit energy table) and merges the range into *d_state and d_xList
- * (capacity cap) with the reference's list rule; asynchronous, no host
- * read-back.  The scratch arrays hold maxBlocks entries; the range may span at
- * most maxBlocks units of 2^(L + lgR) candidates. */
+/* The tables of the low bits' energies and cross sums, kBFTableDoubles
+ * doubles, from W (N x N double); once per search. */
+constexpr int kBFTableDoubles = 32 * 128 + 32 * 32 + 32 * 128 + 32;
+void bfTables(const double *d_W, const BFPlan &p, double *d_tab, hipStream_t stream);
+
+/* Scans x in [xb, xe) (E = x^T W x with W: N x N double) and merges the range
+ * into *d_state and d_xList (capacity cap) with the reference's list rule;
+ * asynchronous, no host read-back.  The scratch arrays hold maxUnits entries;
+ * the range may touch at most maxUnits units.  xb is a multiple of 32, xe too
+ * or 2^N. */
 template <class real>
-void bfSearchRange(const double *d_W, const double *d_EL, const BFPlan &p, unsigned long long xb,
-                   unsigned long long xe, BFState<real> *d_state, unsigned long long cap, real *d_blockMin,
-                   unsigned *d_blockCnt, unsigned long long *d_offsets, int maxBlocks,
-                   unsigned long long *d_xList, hipStream_t stream);
+void bfSearchRange(const double *d_W, const double *d_tab, const BFPlan &p, unsigned long long xb,
+                   unsigned long long xe, BFState<real> *d_state, unsigned long long cap, real *d_unitMin,
+                   unsigned *d_hits, unsigned long long *d_slots, int maxUnits, unsigned long long *d_xList,
+                   hipStream_t stream);
 
 /* The dense search with the caller's device buffers and a static scratch
  * array (bf_noalloc.hip): W real N x N, results Emin (real, sign of the

@@ -425,16 +425,16 @@ private:
     std::vector<double> W_; /* N x N, negated for maximize (:37-38) */
     BFPlan plan_{};
     unsigned long long x_ = 0, xMax_ = 0, span_ = 0;
-    int maxBlocks_ = 0;
+    int maxUnits_ = 0;
     real Emin_ = 0;
     std::vector<unsigned long long> xList_;
     std::vector<real> E_;
 
-    DevBuf<double> d_W_, d_EL_;
+    DevBuf<double> d_W_, d_tab_;
     DevBuf<BFState<real>> d_state_;
-    DevBuf<real> d_blockMin_;
-    DevBuf<unsigned> d_blockCnt_;
-    DevBuf<unsigned long long> d_offsets_, d_xList_;
+    DevBuf<real> d_unitMin_;
+    DevBuf<unsigned> d_hits_;
+    DevBuf<unsigned long long> d_slots_, d_xList_;
 };
 
 /* ------------------------------------------------------------------ */

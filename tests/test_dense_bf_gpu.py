@@ -160,3 +160,31 @@ def test_problem_size_limits(rocm):
     assert s.get_problem_size() == 63
     with pytest.raises(RuntimeError):
         rocm.dense_graph_bf_searcher(dense_int_W(100, SEED_BASE + 100), dtype=np.float32)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("N", [2, 4, 6, 10, 11, 14, 18, 22, 23])
+def test_tied_minimisers_at_unit_sizes(oracle, rocm, dtype, N):
+    """Couplings in [-1, 1] (many ties) at the sizes where the bits run out
+    (rows of 32, 64 rows, 1 to 8 values of c) and where units grow."""
+    W = dense_int_W(N, SEED_BASE + 900 + N, lo=-1, hi=1).astype(dtype)
+    W[0, :] = W[:, 0] = 0  # the top bit is free: every minimiser twice, in two units where there are two
+    _, E, x = search(rocm, W, dtype)
+    Eo, xo = oracle.dense_bf_search(W.astype(np.float64), dtype=dtype)
+    assert float(E[0]) == Eo and packed(x).tolist() == xo.tolist()
+
+
+def test_span_cut_inside_a_unit(rocm):
+    """A tile size that is no multiple of a unit: the spans meet inside one.
+    E = -x[0] - x[N-1]: the odd x of the upper half."""
+    N, tile = 27, (1 << 26) + 256
+    W = np.zeros((N, N), np.float32)
+    W[0, 0] = W[N - 1, N - 1] = -1.0
+    s = rocm.dense_graph_bf_searcher(W, dtype=np.float32, tile_size=tile)
+    s.prepare()
+    assert s.search_range() == (False, tile)
+    assert s.search_range() == (True, 1 << N)
+    s.make_solution()
+    p = packed(np.array(s.get_x()[:5000], np.int8))
+    assert np.all(s.get_E() == -2.0) and len(s.get_E()) == 1 << 25
+    assert p.tolist() == [(1 << 26) + 2 * i + 1 for i in range(5000)]
