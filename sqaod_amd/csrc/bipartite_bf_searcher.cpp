@@ -10,8 +10,8 @@
  * first N0 + N1 pairs reaching it in one worker's visiting order (x0 tile,
  * x1, x0 within the tile; CPUBipartiteGraphBatchSearch.cpp:47-60) -- the
  * one-worker CPU result.  Each searchRange scans a rectangle of x1 values
- * times high-x0 patterns; the device returns each block's first minimisers
- * and the host merges them by visiting key, so the result does not depend on
+ * times high-x0 patterns; the device returns the first minimisers of each x1
+ * and 16 high patterns and the host merges them by visiting key, so the result does not depend on
  * how the pairs were cut into rectangles.
  */
 #include <algorithm>
@@ -23,7 +23,8 @@
 namespace sqaod_rocm {
 
 namespace {
-constexpr unsigned long long kMaxBlocks = 1ull << 15; /* blocks per rectangle (each 16 x 2^L pairs) */
+constexpr unsigned long long kMaxItems = 1ull << 15; /* items per rectangle (each 16 x 2^L pairs) */
+constexpr unsigned long long kFirstPairs = 64;       /* pairs read back with their number */
 }  // namespace
 
 template <class real>
@@ -109,17 +110,20 @@ void BipartiteGraphBFSearcher<real>::prepare() {
     T0_ = std::min<unsigned long long>((unsigned long long)tileSize0_, 1ull << N0_);
     plan_ = bgBFPlan(N0_, N1_);
     plan_.sgn = (om_ == optMaximize) ? -1. : 1.;
-    /* rectangles: up to 4096 x1 values times enough high patterns for kMaxBlocks blocks */
+    /* rectangles: up to 4096 x1 values times enough high patterns for kMaxItems items */
     x1Chunk_ = std::min<unsigned long long>(1ull << N1_, 4096);
     const unsigned long long nHigh = 1ull << plan_.nH;
-    hChunk_ = std::min<unsigned long long>(nHigh, std::max<unsigned long long>(1, kMaxBlocks / x1Chunk_) *
+    hChunk_ = std::min<unsigned long long>(nHigh, std::max<unsigned long long>(1, kMaxItems / x1Chunk_) *
                                                       (unsigned long long)kBGBFHighPerBlock);
     hNext_ = 0;
     x1Next_ = 0;
-    const unsigned long long blocks = x1Chunk_ * ((hChunk_ + kBGBFHighPerBlock - 1) / kBGBFHighPerBlock);
-    d_blockMin_.allocate(blocks);
-    d_counts_.allocate(blocks);
-    d_pairs_.allocate(blocks * 2 * (size_t)plan_.K);
+    const unsigned long long items = x1Chunk_ * ((hChunk_ + kBGBFHighPerBlock - 1) / kBGBFHighPerBlock);
+    d_x1Min_.allocate(x1Chunk_);
+    d_pairs_.allocate(2 + items * 2 * (size_t)plan_.K);
+    h_pairs_.allocate(2 + 2 * kFirstPairs);
+    h_blockMin_.allocate((size_t)((x1Chunk_ + kBGBFScanBlock - 1) / kBGBFScanBlock),
+                         hipHostMallocCoherent | hipHostMallocMapped);
+    HIP_CHECK(hipHostGetDevicePointer((void **)&d_blockMin_, h_blockMin_.ptr, 0));
     setState(solPrepared);
 }
 
@@ -135,37 +139,38 @@ bool BipartiteGraphBFSearcher<real>::searchRange(unsigned long long *curX0, unsi
         a.he = std::min(hNext_ + hChunk_, nHigh);
         a.x1b = x1Next_;
         a.nX1 = std::min(x1Chunk_, x1max - x1Next_);
-        const unsigned long long blocks = bgBFBlocks(a);
         hipStream_t st = dev_->stream();
-        bgBFScan<real>(a, d_b0_.ptr, d_b1_.ptr, d_W_.ptr, d_blockMin_.ptr, st);
-        std::vector<real> bm(blocks);
-        HIP_CHECK(hipMemcpyAsync(bm.data(), d_blockMin_.ptr, blocks * sizeof(real), hipMemcpyDeviceToHost, st));
+        bgBFScan<real>(a, d_b0_.ptr, d_b1_.ptr, d_W_.ptr, d_x1Min_.ptr, d_blockMin_, d_pairs_.ptr, st);
         HIP_CHECK(hipStreamSynchronize(st));
-        const real rmin = *std::min_element(bm.begin(), bm.end());
+        const real rmin = *std::min_element(h_blockMin_.ptr, h_blockMin_.ptr + bgBFScanBlocks(a));
         if (rmin <= Emin_) {
             if (rmin < Emin_) {
                 Emin_ = rmin;
                 list_.clear();
             }
-            bgBFSelect<real>(a, d_b0_.ptr, d_b1_.ptr, d_W_.ptr, d_blockMin_.ptr, rmin, d_pairs_.ptr, d_counts_.ptr,
+            bgBFSelect<real>(a, d_b0_.ptr, d_b1_.ptr, d_W_.ptr, d_x1Min_.ptr, rmin, d_pairs_.ptr + 2, d_pairs_.ptr,
                              st);
-            std::vector<int> cnt(blocks);
-            HIP_CHECK(hipMemcpyAsync(cnt.data(), d_counts_.ptr, blocks * sizeof(int), hipMemcpyDeviceToHost, st));
+            const size_t room = std::min<size_t>(h_pairs_.n, d_pairs_.n);
+            HIP_CHECK(hipMemcpyAsync(h_pairs_.ptr, d_pairs_.ptr, room * sizeof(unsigned long long),
+                                     hipMemcpyDeviceToHost, st));
             HIP_CHECK(hipStreamSynchronize(st));
-            const size_t K = (size_t)plan_.K;
-            std::vector<unsigned long long> buf(2 * K);
+            const size_t n = (size_t)h_pairs_.ptr[0];
+            const unsigned long long *pairs = h_pairs_.ptr + 2;
+            std::vector<unsigned long long> all;
+            if (2 + 2 * n > room) {
+                all.resize(2 * n);
+                HIP_CHECK(hipMemcpyAsync(all.data(), d_pairs_.ptr + 2, 2 * n * sizeof(unsigned long long),
+                                         hipMemcpyDeviceToHost, st));
+                HIP_CHECK(hipStreamSynchronize(st));
+                pairs = all.data();
+            }
             std::vector<std::pair<unsigned long long, std::pair<unsigned long long, unsigned long long>>> cand;
             for (auto &p : list_)
                 cand.push_back({visitKey(p.first, p.second), p});
-            for (unsigned long long b = 0; b < blocks; ++b) {
-                if (cnt[b] == 0)
-                    continue;
-                HIP_CHECK(hipMemcpy(buf.data(), d_pairs_.ptr + b * 2 * K, (size_t)cnt[b] * 2 * sizeof(unsigned long long),
-                                    hipMemcpyDeviceToHost));
-                for (int k = 0; k < cnt[b]; ++k)
-                    cand.push_back({visitKey(buf[2 * k], buf[2 * k + 1]), {buf[2 * k], buf[2 * k + 1]}});
-            }
+            for (size_t k = 0; k < n; ++k)
+                cand.push_back({visitKey(pairs[2 * k], pairs[2 * k + 1]), {pairs[2 * k], pairs[2 * k + 1]}});
             std::sort(cand.begin(), cand.end());
+            const size_t K = (size_t)plan_.K;
             list_.clear();
             for (size_t k = 0; k < cand.size() && k < K; ++k)
                 list_.push_back(cand[k].second);

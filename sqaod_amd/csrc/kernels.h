@@ -347,16 +347,20 @@ struct BGBFArgs {
     unsigned long long x1b, nX1, hb, he;
 };
 BGBFArgs bgBFPlan(int N0, int N1);
-unsigned long long bgBFBlocks(const BGBFArgs &a);
-/* blockMin[bgBFBlocks(a)]: each block's minimum E */
+constexpr int kBGBFScanBlock = 64;
+unsigned long long bgBFItems(const BGBFArgs &a);      /* (x1, 16 high patterns) of the rectangle */
+unsigned long long bgBFScanBlocks(const BGBFArgs &a);
+/* x1Min[nX1]: each x1's least E over the rectangle's x0 (at most FLT_MAX);
+ * blockMin[bgBFScanBlocks(a)] (host-visible memory): the least of each 64;
+ * *nPairs is set to 0 */
 template <class real>
-void bgBFScan(const BGBFArgs &a, const real *d_b0, const real *d_b1, const real *d_W, real *d_blockMin,
-              hipStream_t stream);
-/* blocks whose minimum is Emin write their first K minimisers (ascending x0,
- * pairs (x0, x1) as 2 u64) to pairs[block * 2K ...] and the count to counts[block] */
+void bgBFScan(const BGBFArgs &a, const real *d_b0, const real *d_b1, const real *d_W, real *d_x1Min,
+              real *d_blockMin, unsigned long long *d_nPairs, hipStream_t stream);
+/* each item whose x1 reaches Emin appends its first K minimisers (ascending
+ * x0, pairs (x0, x1) as 2 u64) to pairs (bgBFItems(a) * K pairs), *nPairs in all */
 template <class real>
-void bgBFSelect(const BGBFArgs &a, const real *d_b0, const real *d_b1, const real *d_W, const real *d_blockMin,
-                real Emin, unsigned long long *d_pairs, int *d_counts, hipStream_t stream);
+void bgBFSelect(const BGBFArgs &a, const real *d_b0, const real *d_b1, const real *d_W, const real *d_x1Min,
+                real Emin, unsigned long long *d_pairs, unsigned long long *d_nPairs, hipStream_t stream);
 
 /* ---------------- energies (energy.hip) ---------------- */
 

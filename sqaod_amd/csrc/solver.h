@@ -477,9 +477,11 @@ private:
     real Emin_ = 0;
     std::vector<std::pair<unsigned long long, unsigned long long>> list_; /* (x0, x1), visiting order */
     std::vector<real> E_;
-    DevBuf<real> d_b0_, d_b1_, d_W_, d_blockMin_;
-    DevBuf<unsigned long long> d_pairs_;
-    DevBuf<int> d_counts_;
+    DevBuf<real> d_b0_, d_b1_, d_W_, d_x1Min_;
+    DevBuf<unsigned long long> d_pairs_; /* the number of pairs (2 words), then the pairs */
+    PinnedBuf<real> h_blockMin_;
+    PinnedBuf<unsigned long long> h_pairs_;
+    real *d_blockMin_ = nullptr; /* h_blockMin_ as the device sees it */
 };
 
 /* ------------------------------------------------------------------ */

@@ -94,3 +94,30 @@ def test_errors(rocm):
         s.set_qubo(np.ones(3), np.ones(2), np.ones((3, 2)))
     with pytest.raises(RuntimeError):
         s.prepare()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("N0,N1", [(1, 1), (63, 1), (11, 5), (4, 12), (20, 1), (18, 13)])
+def test_real_weights_take_the_least_over_x0(rocm, dtype, N0, N1):
+    """N(0, 1) weights, where the minimum is one pair: the x0 of the negative
+    sums of its x1, over one to many rectangles of high patterns (N0 = 63: the
+    first rectangle alone, its high bits fixed at zero)."""
+    rng = np.random.default_rng(SEED_BASE + 100 * N0 + N1)
+    b0, b1, W = (rng.standard_normal(s).astype(dtype) for s in (N0, N1, (N1, N0)))
+    s = rocm.bipartite_graph_bf_searcher(b0, b1, W, dtype=dtype)
+    s.prepare()
+    done, cx0, _ = s.search_range()
+    while not done and N0 <= 20:
+        done, cx0, _ = s.search_range()
+    s.make_solution()
+    x1 = ((np.arange(1 << N1)[:, None] >> np.arange(N1 - 1, -1, -1)) & 1).astype(np.float64)
+    d = b0.astype(np.float64) + x1 @ W.astype(np.float64)
+    if N0 == 63:
+        d[:, packed(np.eye(N0, dtype=np.uint64)) >= cx0] = 0.0  # not reached
+    E = np.minimum(d, 0.0).sum(axis=1) + x1 @ b1.astype(np.float64)
+    best = int(np.argmin(E))
+    x = s.get_x()
+    assert len(x) == 1 and packed(x[0][1]) == best and np.array_equal(np.asarray(x[0][0]), (d[best] < 0).astype(np.int8))
+    # (N0 + 1)(N1 + 1) terms summed in 64 bits in two orders, then one rounding to dtype
+    sums = 2 * (N0 + 1) * (N1 + 1) * 2.0 ** -53 * sum(np.abs(v.astype(np.float64)).sum() for v in (b0, b1, W))
+    assert abs(float(s.get_E()[0]) - E[best]) <= sums + np.finfo(dtype).eps / 2 * (abs(E[best]) + sums)
