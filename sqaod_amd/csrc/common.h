@@ -47,8 +47,8 @@ struct Error : std::runtime_error {
                                       hipGetErrorString(e_), #expr);                          \
     } while (0)
 
-inline int divru(int a, int b) { return (a + b - 1) / b; }
-inline int roundUp(int a, int b) { return divru(a, b) * b; }
+__host__ __device__ inline int divru(int a, int b) { return (a + b - 1) / b; }
+__host__ __device__ inline int roundUp(int a, int b) { return divru(a, b) * b; }
 
 /* Device memory owned by a solver; freed in the destructor. */
 template <class T>

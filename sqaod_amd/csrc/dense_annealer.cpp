@@ -395,9 +395,10 @@ void DenseGraphAnnealer<real>::setPreference(const std::string &name, const std:
             multiFlipMin_ = v;
         }
     } else if (name == "helper_wave") {
-        /* "on" (default): single-flip float local-field sweeps with one slice
-         * per block run a second wave per slice that applies the deferred J
-         * rows to the fields; "off": the sweeping wave applies them */
+        /* "on" (default): single-flip local-field sweeps run by a team of
+         * four waves per slice, one deciding, one adding the flipped spins' J
+         * rows to the fields, one preparing the attempts ahead, one reading the
+         * neighbour slices' decisions; "off": one wave per slice does it all */
         if (value == "on" || value == "true" || value == "True" || value == "1")
             helperWave_ = true;
         else if (value == "off" || value == "false" || value == "False" || value == "0")
@@ -596,6 +597,9 @@ void DenseGraphAnnealer<real>::prepare() {
     d_D_.allocate(mN);
     HIP_CHECK(hipMemsetAsync(d_Q_.ptr, 0, d_Q_.bytes(), dev_->stream()));
     HIP_CHECK(hipMemsetAsync(d_D_.ptr, 0, d_D_.bytes(), dev_->stream()));
+    ldP_ = teamWordStride(N_);
+    d_P_.allocate((size_t)m_ * ldP_);
+    HIP_CHECK(hipMemsetAsync(d_P_.ptr, 0, d_P_.bytes(), dev_->stream()));
     tag_ = 0;
     d_E_.allocate((size_t)m_);
     ensureEnergyPlanes();
@@ -796,6 +800,8 @@ SweepArgs<real> DenseGraphAnnealer<real>::makeSweepArgs(real G, real beta) {
     a.D = d_D_.ptr;
     reserveTags(1);
     a.tag = ++tag_;
+    a.P = d_P_.ptr;
+    a.ldP = ldP_;
     a.abortFlag = d_abort_.ptr;
     a.abortHost = d_abortHost_;
     a.counters = d_counters_.ptr;
@@ -908,20 +914,22 @@ void DenseGraphAnnealer<real>::annealOneStep(real G, real beta) {
         if (a.multiBufs >= 2)
             sweepFormat = f;
     }
-    /* the helper-wave sweep where it fits; the fp8 form's runs on the float
-     * copy of J' as well (the same row values, -+2 J'[x][s]) */
-    if (helperWave_ && a.multiBufs < 2) {
-        const int f = sweepFormat == fieldFP8 ? fieldF32 : sweepFormat;
-        if (denseSweepHelperFits(Np_, S, sizeof(real), plainSweep_, f, dev_->maxLdsPerBlock())) {
-            a.helperWave = 1;
-            sweepFormat = f;
-        }
-    }
     ++sweepsSinceSpinsSet_;
+    const bool direct = !coopLaunch_ && dev_->soleSweeper();
     if (profile_)
         phaseBegin(2, pe);
-    denseSweep<real>(a, plainSweep_, sweepFormat, S, !coopLaunch_ && dev_->soleSweeper(), dev_->numCUs(),
-                     dev_->stream());
+    /* the team sweep where it fits; the fp8 form's runs on the float copy of J'
+     * (a.J) as well */
+    int teamS = 0;
+    if (helperWave_ && !plainSweep_ && a.multiBufs < 2)
+        teamS = denseSweepTeamSlices(N_, Np_, m_, sizeof(real), slicesPerBlock_, dev_->numCUs(), dev_->maxLdsPerBlock());
+    if (teamS > 0) {
+        if (a.tag % kTeamTagPeriod == 0) /* its words' tags start over */
+            HIP_CHECK(hipMemsetAsync(d_P_.ptr, 0, d_P_.bytes(), dev_->stream()));
+        denseSweepTeam<real>(a, teamS, dev_->maxLdsPerBlock(), direct, dev_->numCUs(), dev_->stream());
+    } else {
+        denseSweep<real>(a, plainSweep_, sweepFormat, S, direct, dev_->numCUs(), dev_->stream());
+    }
     if (profile_)
         phaseEnd(pe);
     if (pending_.size() > 3000)

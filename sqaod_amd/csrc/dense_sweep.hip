@@ -28,24 +28,19 @@
  * cycle and all waves finish; a spin limit turns a bug into an error instead
  * of a hang.  All waves must be co-resident (see denseSweep's launch).
  */
-#include "common.h"
-#include "kernels.h"
-#include "sq_expf.h"
+#include "sweep_device.h"
 
 #include <map>
 #include <mutex>
 #include <tuple>
-#include <type_traits>
 
 namespace sqaod_rocm {
 
 namespace {
 
-constexpr int kWave = 64;
 constexpr int kTblMax = 4096; /* entries of the pending-site table per slice */
 constexpr int kDotGroup = 8; /* plain sweep: attempts whose dots are formed together */
 constexpr int kMaxSlicesPerBlock = 4; /* one wave per SIMD, so a wave may hold up to 256 VGPRs */
-constexpr size_t kExpTabBytes = 32 * sizeof(uint64_t); /* LDS copy of the exp table */
 
 /* Optional per-phase cycle counters (build with -DSQAOD_SWEEP_CYCLES): shader
  * clock cycles spent per phase, summed into SweepArgs::counters[3..15]. */
@@ -60,82 +55,9 @@ constexpr size_t kExpTabBytes = 32 * sizeof(uint64_t); /* LDS copy of the exp ta
 #endif
 
 
-__device__ __forceinline__ uint32_t loadShared32(const uint32_t *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void storeShared32(uint32_t *p, uint32_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
-__device__ __forceinline__ void waveSync() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-__device__ __forceinline__ int firstLane(unsigned long long mask) {
-    return mask ? (int)__builtin_ctzll(mask) : kWave;
-}
-
-/* lane l's float (l wave-uniform) */
-__device__ __forceinline__ float readLaneF(float v, int l) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-
-/* A wave-uniform int, marked so: control values the compiler cannot prove
- * uniform (they pass through loops with ballot-dependent exits) would
- * otherwise live in VGPRs and turn every branch on them into exec masking. */
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-
-/* LDS DMA issued from inline assembly: lane i's 4 (16) bytes from src land at
- * ldsDst + 4i (16i).  The compiler sees neither the op nor its LDS write, so
- * it adds no memory waits for it (for the builtin form it waits for every
- * outstanding DMA before any later LDS access, which serialises the batch
- * loop); every read of a DMA destination follows an explicit vmWait instead.
- * Ops the compiler does not count only make its own waits stricter (vmcnt
- * retires in issue order), never weaker.  M0 carries the LDS address; nothing
- * else in the sweep kernels uses M0.  kCoherent: the cache policy of a relaxed
- * atomic load at agent scope (decisions published by other waves). */
-/* the M0 clobber below is deliberate (clang warns about any M0 clobber) */
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ uint32_t ldsAddress(const void *p) {
-    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p);
-}
-template <bool kCoherent>
-__device__ __forceinline__ void dmaDword(const void *src, uint32_t lds) {
-    const uint32_t m = __builtin_amdgcn_readfirstlane(lds);
-    if constexpr (kCoherent)
-        asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off sc1" ::"v"(src), "s"(m) : "memory", "m0");
-    else
-        asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(m) : "memory", "m0");
-}
-__device__ __forceinline__ void dmaDwordx4(const void *src, uint32_t lds) {
-    const uint32_t m = __builtin_amdgcn_readfirstlane(lds);
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m) : "memory", "m0");
-}
-/* n consecutive 1 KiB DMA ops (16 B per lane): op i reads src + i KiB (src:
- * this lane's address for op 0) and lands at LDS byte address lds + i KiB.
- * Groups of four set M0 once and step it by 1 KiB (a wait state after each
- * M0 write before the DMA reads it). */
-__device__ __forceinline__ void dmaRunx4(const unsigned char *src, uint32_t lds, int n) {
-    int i = 0;
-    for (; i + 4 <= n; i += 4) { /* n is wave-uniform: a scalar loop */
-        const uint32_t m = __builtin_amdgcn_readfirstlane(lds + (uint32_t)i * 1024u);
-        const unsigned char *p = src + (size_t)i * 1024;
-        asm volatile("s_mov_b32 m0, %4\n\ts_nop 0\n\t"
-                     "global_load_lds_dwordx4 %0, off\n\t"
-                     "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
-                     "global_load_lds_dwordx4 %1, off\n\t"
-                     "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
-                     "global_load_lds_dwordx4 %2, off\n\t"
-                     "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
-                     "global_load_lds_dwordx4 %3, off" ::"v"(p),
-                     "v"(p + 1024), "v"(p + 2048), "v"(p + 3072), "s"(m)
-                     : "memory", "m0", "scc");
-    }
-    for (; i < n; ++i)
-        dmaDwordx4(src + (size_t)i * 1024, lds + (uint32_t)i * 1024u);
-}
 /* A neighbour's two 128-entry windows when all their entries lie in its row:
  * the decisions (coherent loads) at LDS byte address lds and the sites 1 KiB
  * above it, 256 B per op, four ops on one M0 chain.  d, x: this lane's entry
@@ -155,53 +77,6 @@ __device__ __forceinline__ void dmaNeighbourWindows(const uint32_t *d, const uin
 }
 #pragma clang diagnostic pop
 
-/* wait until at most C vector-memory ops are outstanding */
-template <int C>
-__device__ __forceinline__ void vmWaitImm() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C) : "memory");
-}
-template <int LO, int HI>
-__device__ __forceinline__ void vmWaitRange(int c) {
-    if constexpr (LO == HI) {
-        vmWaitImm<LO>();
-    } else {
-        constexpr int MID = (LO + HI + 1) / 2;
-        if (c >= MID)
-            vmWaitRange<MID, HI>(c);
-        else
-            vmWaitRange<LO, MID - 1>(c);
-    }
-}
-/* vmcnt(c) for a wave-uniform c (counts above 63 wait for 63) */
-__device__ __forceinline__ void vmWait(int c) {
-    c = __builtin_amdgcn_readfirstlane(c);
-    if (c == 1) /* the common case: only a decision store since */
-        vmWaitImm<1>();
-    else
-        vmWaitRange<0, 63>(c < 63 ? c : 63);
-}
-/* this wave's LDS reads have returned (before a DMA overwrites what they read) */
-__device__ __forceinline__ void ldsWait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
-/* Copy kEntries entries of ES bytes, from entry e0 of src, into LDS at lds by
- * DMA, skipping entries >= limit (their LDS words keep old contents). */
-template <int ES, bool kCoherent, int kEntries>
-__device__ __forceinline__ void dmaEntries(const void *src, uint32_t lds, int e0, int limit) {
-    const int lane = threadIdx.x & (kWave - 1);
-    constexpr int kOps = kEntries * ES / (4 * kWave);
-    const uint32_t *s = reinterpret_cast<const uint32_t *>(src) + lane;
-    if (e0 + kEntries <= limit) {
-#pragma unroll
-        for (int j = 0; j < kOps; ++j)
-            dmaDword<kCoherent>(s + j * kWave, lds + j * kWave * 4);
-    } else {
-#pragma unroll
-        for (int j = 0; j < kOps; ++j)
-            if (e0 + (j * kWave + lane) * 4 / ES < limit)
-                dmaDword<kCoherent>(s + j * kWave, lds + j * kWave * 4);
-    }
-}
-
 /* entries of the per-slice pending-site table: a power of two >= min(Np, 4096);
  * sites are hashed by their low bits, a collision only delays a lane. */
 __host__ __device__ inline int pendingTableSize(int Np) {
@@ -220,11 +95,6 @@ constexpr int kPendMulti = 1 << 30;
 __device__ __forceinline__ int pendCode(int rel, int N, int nb) { return ((rel + N) << 1) | nb; }
 __device__ __forceinline__ int pendRel(int code, int N) { return ((code & (kPendMulti - 1)) >> 1) - N; }
 
-__device__ __forceinline__ int slicePos(int y, int m) {
-    int nEven = (m + 1) / 2;
-    return (y & 1) ? nEven + (y >> 1) : (y >> 1);
-}
-
 /* 4 consecutive elements of a J row (16- or 32-byte vector load). */
 template <class real>
 __device__ __forceinline__ void loadJ4(const real *p, real v[4]) {
@@ -238,51 +108,9 @@ __device__ __forceinline__ void loadJ4(const real *p, real v[4]) {
     }
 }
 
-template <class real>
-__device__ __forceinline__ void ldsLoad4(const real *p, real v[4]) {
-    if constexpr (sizeof(real) == 4) {
-        float4 t = *reinterpret_cast<const float4 *>(p);
-        v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
-    } else {
-        double2 t0 = *reinterpret_cast<const double2 *>(p);
-        double2 t1 = *reinterpret_cast<const double2 *>(p + 2);
-        v[0] = t0.x; v[1] = t0.y; v[2] = t1.x; v[3] = t1.y;
-    }
-}
-
-template <class real>
-__device__ __forceinline__ void ldsStore4(real *p, const real v[4]) {
-    if constexpr (sizeof(real) == 4) {
-        *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
-    } else {
-        *reinterpret_cast<double2 *>(p) = make_double2(v[0], v[1]);
-        *reinterpret_cast<double2 *>(p + 2) = make_double2(v[2], v[3]);
-    }
-}
-
-template <class real>
-struct Expo;
-template <>
-struct Expo<float> {
-    /* the CPU annealer's expf(-dE*beta), bit-identical (sq_expf.h) */
-    __device__ static float eval(float v, const uint64_t *tab) { return sq_expf_tab(v, tab); }
-};
-template <>
-struct Expo<double> {
-    __device__ static double eval(double v, const uint64_t *) { return exp(v); }
-};
-
 /* Kernel variants: local fields with rows of args.J, the plain reference
  * algorithm, and local fields with the fp8 rows of args.J8 (float only). */
 enum SweepMode { kModeLocal = 0, kModePlain = 1, kModeFP8 = 2 };
-
-/* 4 e4m3 bytes -> floats (exact), gfx950's OCP FP8 conversion */
-__device__ __forceinline__ void fp8x4ToFloat(uint32_t w, float v[4]) {
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, false);
-    const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, true);
-    v[0] = lo.x; v[1] = lo.y; v[2] = hi.x; v[3] = hi.y;
-}
 
 /* Fixed part of a wave's LDS region: the two neighbour windows (decisions and
  * sites of kWin entries each), the own-stream ring (sites and uniforms of
@@ -308,23 +136,12 @@ __host__ __device__ constexpr bool multiFlipCapable() {
     return MODE == kModeLocal && sizeof(real) == 4;
 }
 
-/* Helper wave (float local-field sweep, one slice per workgroup): a second
- * row stage buffer and the command word the two waves exchange. */
-constexpr size_t kHelperCtlBytes = 256;
-constexpr int kHelperRounds = 4; /* the helper's row add: 256-element slices in flight */
-
-template <class real, int MODE>
-__host__ __device__ constexpr bool helperCapable() {
-    return MODE == kModeLocal && sizeof(real) == 4;
-}
-
 /* Bytes of LDS one wave's slice needs (the fixed part, fields, row stage,
  * pending table, spin bits and the two mirrors), for a row length Np; with
  * multiBufs >= 2 also multiBufs - 1 more row stage buffers and the
- * submatrix of multi-flip batches; with helper (helperCapable forms) a
- * second row stage buffer and the helper's command word. */
+ * submatrix of multi-flip batches. */
 template <class real, int MODE>
-__host__ __device__ inline size_t sweepWaveBytes(int Np, int ld8, int multiBufs = 0, bool helper = false) {
+__host__ __device__ inline size_t sweepWaveBytes(int Np, int ld8, int multiBufs = 0) {
     constexpr bool PLAIN = MODE == kModePlain;
     constexpr bool FP8 = MODE == kModeFP8;
     constexpr bool kDefer = !PLAIN && sizeof(real) == 4;
@@ -333,88 +150,7 @@ __host__ __device__ inline size_t sweepWaveBytes(int Np, int ld8, int multiBufs 
     size_t b = sweepFixedBytes<real>() + fieldBytes + (size_t)pendingTableSize(Np) * 4 + (size_t)3 * (Np / 32) * 4;
     if (multiFlipCapable<real, MODE>() && multiBufs >= 2)
         b += (size_t)(multiBufs - 1) * stageBytes + kSubBytes;
-    else if (helperCapable<real, MODE>() && helper)
-        b += stageBytes + kHelperCtlBytes;
     return b;
-}
-
-/* Helper-wave commands (the word at the end of the slice's region): the
- * sweeping wave writes "apply buffer b with factor -+2" once the row has
- * landed in LDS (its own vmcnt wait); the helper adds the row to F, waits for
- * its LDS stores and writes kHelpIdle; kHelpExit ends it.  The word is read
- * and written with relaxed LDS atomics: a wave's LDS operations execute in
- * issue order, and the compiler barriers around them keep the field accesses
- * on their side of the exchange. */
-constexpr uint32_t kHelpIdle = 0, kHelpExit = 1;
-__device__ __forceinline__ uint32_t helpApply(int buf, bool negative) {
-    return 2u + ((uint32_t)buf << 1) + (negative ? 1u : 0u);
-}
-__device__ __forceinline__ uint32_t helpLoad(const uint32_t *ctl) {
-    const uint32_t v = __hip_atomic_load(ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    asm volatile("" ::: "memory");
-    return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
-}
-__device__ __forceinline__ void helpStore(uint32_t *ctl, uint32_t v) {
-    asm volatile("" ::: "memory");
-    if ((threadIdx.x & (kWave - 1)) == 0)
-        __hip_atomic_store(ctl, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-/* the slice region's helper command word: after the second stage buffer,
- * which follows the spin bits and mirrors */
-template <class real>
-__device__ __forceinline__ uint32_t *helperCtl(const SweepArgs<real> &a, unsigned char *p) {
-    const size_t stageBytes = (size_t)a.Np * sizeof(real);
-    unsigned char *body = p + sweepFixedBytes<real>();
-    unsigned char *bits = body + (size_t)a.Np * sizeof(real) + stageBytes + (size_t)pendingTableSize(a.Np) * 4;
-    unsigned char *buf1 = bits + (size_t)3 * a.Nw * 4;
-    return reinterpret_cast<uint32_t *>(buf1 + stageBytes);
-}
-
-/* f + d * v for a field update: d is -+2 (fp8 rows: -+2 times the row's
- * power-of-two scale) and v a J element, so d * v is exact and one fused
- * multiply-add rounds exactly as the separate multiply and add do. */
-__device__ __forceinline__ float addScaled(float f, float d, float v) { return __builtin_fmaf(d, v, f); }
-__device__ __forceinline__ double addScaled(double f, double d, double v) { return __builtin_fma(d, v, f); }
-
-/* F[b0 ..] += d * sb[b0 ..] for R consecutive 256-element slices: all their
- * LDS reads are issued before the first write, so the round trips overlap.
- * FP8: sb holds e4m3 bytes. */
-template <class real, bool FP8, int R>
-__device__ __forceinline__ void addStagedSlices(real *F, const real *sb, real d, int b0, int lane) {
-#pragma clang fp contract(off)
-    const uint8_t *sb8 = reinterpret_cast<const uint8_t *>(sb);
-    (void)sb8;
-    real fv[R][4], sv[R][4];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int j = b0 + r * kWave * 4 + lane * 4;
-        ldsLoad4(F + j, fv[r]);
-        if constexpr (FP8)
-            fp8x4ToFloat(*reinterpret_cast<const uint32_t *>(sb8 + j), sv[r]);
-        else
-            ldsLoad4(sb + j, sv[r]);
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int j = b0 + r * kWave * 4 + lane * 4;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            fv[r][t] = addScaled(fv[r][t], d, sv[r][t]);
-        ldsStore4(F + j, fv[r]);
-    }
-}
-
-/* F += d * (staged row sb): rounds of kR 256-element slices, then single
- * slices for the rest (Np is a multiple of 256).  The rounds carry no
- * per-slice bounds checks, so their reads go out back to back. */
-template <class real, bool FP8, int kR = 4>
-__device__ __forceinline__ void addStagedRow(real *F, const real *sb, real d, int Np, int lane) {
-    int b0 = 0;
-    /* b0 and the bounds are wave-uniform: scalar loops */
-    for (; b0 + kR * kWave * 4 <= Np; b0 += kR * kWave * 4)
-        addStagedSlices<real, FP8, kR>(F, sb, d, b0, lane);
-    for (; b0 < Np; b0 += kWave * 4)
-        addStagedSlices<real, FP8, 1>(F, sb, d, b0, lane);
 }
 
 /* F += d[0] * row 0, then d[1] * row 1, ... (NR rows, in that order per
@@ -453,36 +189,11 @@ __device__ __forceinline__ void addStagedRows(real *F, const real *const *sb, co
         slices(b0, std::integral_constant<int, 1>());
 }
 
-/* The helper wave of a slice (float local-field sweep): waits for commands
- * from the sweeping wave and applies the rows it hands over, F += d * row,
- * with the same per-element operation the sweeping wave would use. */
-template <class real>
-__device__ void helperLoop(const SweepArgs<real> &a, unsigned char *p) {
-    const int Np = a.Np;
-    const int lane = threadIdx.x & (kWave - 1);
-    real *F = reinterpret_cast<real *>(p + sweepFixedBytes<real>());
-    uint32_t *ctl = helperCtl(a, p);
-    real *const buf[2] = {F + Np, reinterpret_cast<real *>(reinterpret_cast<unsigned char *>(ctl) - (size_t)Np * sizeof(real))};
-    for (;;) {
-        const uint32_t c = helpLoad(ctl);
-        if (c == kHelpIdle) {
-            __builtin_amdgcn_s_sleep(1);
-            continue;
-        }
-        if (c == kHelpExit)
-            break;
-        const uint32_t cmd = c - 2u;
-        addStagedRow<real, false, kHelperRounds>(F, buf[cmd >> 1], (cmd & 1u) ? (real)-2. : (real)2., Np, lane);
-        ldsWait(); /* the field stores are done */
-        helpStore(ctl, kHelpIdle);
-    }
-}
-
 /* One wave runs the whole sweep of slice y: N attempts, with its LDS region
  * p (sweepWaveBytes), the exp table and h already in LDS.  MULTI compiles the
  * multi-flip batches in (float local-field form only); without it the batch
  * ends at its first accepted flip. */
-template <class real, int MODE, bool MULTI = false, bool HELPER = false>
+template <class real, int MODE, bool MULTI = false>
 __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y, const uint64_t *expTab,
                                            const real *hS, unsigned char *p) {
 #pragma clang fp contract(off)
@@ -538,16 +249,6 @@ __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y
     };
     (void)stageBuf;
     (void)stageBufL;
-    /* Helper wave: the pending row is handed to the slice's second wave at
-     * the commit instead of being applied there, and the next row streams
-     * into the other of stage buffers 0 and 1.  The handed row must be in F
-     * before the next evaluation reads F (helpBusy: wait for kHelpIdle). */
-    constexpr bool kHelp = HELPER && kDefer && !FP8 && !kMultiCap && helperCapable<real, MODE>();
-    uint32_t *const ctl = reinterpret_cast<uint32_t *>(multiBase + stageBytes);
-    bool helpBusy = false;
-    (void)ctl;
-    (void)helpBusy;
-
     const long long yN = (long long)y * N;
     const int n0 = (y == 0) ? m - 1 : y - 1;
     const int n1 = (y == m - 1) ? 0 : y + 1;
@@ -689,8 +390,7 @@ __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y
 
     /* load wait, neighbours, evaluate, commit, row, blocked; within neighbours:
      * replay and registration, row wait, prefetch issue; within the row:
-     * the pending row's application, the next row's DMA issue; within the
-     * evaluation: the wait for the helper wave; multi-flip commits: the
+     * the pending row's application, the next row's DMA issue; multi-flip commits: the
      * waits for rows applied at once */
     unsigned long long cyc[13] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     (void)cyc;
@@ -909,16 +609,6 @@ __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y
         } else {
             /* decided under both outcomes of the pending attempt: if they
              * agree the decision is final, otherwise the lane waits */
-            if constexpr (kHelp) {
-                if (helpBusy) {
-                    SQ_CYC(h0);
-                    while (helpLoad(ctl) != kHelpIdle)
-                        ;
-                    helpBusy = false;
-                    SQ_CYC(h1);
-                    SQ_CYC_ADD(cyc[11], h0, h1);
-                }
-            }
             real f = F[s];
             if constexpr (kMultiCap) {
 #pragma unroll
@@ -1116,13 +806,6 @@ __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y
         if constexpr (kMultiCap) {
             if (nPend > 0)
                 applyPendingRows();
-        } else if constexpr (kHelp) {
-            if (rowPending) {
-                /* the row landed before this batch's evaluation (vmcnt) */
-                helpStore(ctl, helpApply(curStage, rowD < (real)0.));
-                helpBusy = true;
-                rowPending = false;
-            }
         } else if constexpr (kDefer) {
             if (rowPending)
                 applyPendingRow();
@@ -1130,8 +813,8 @@ __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y
         SQ_CYC(r1);
         SQ_CYC_ADD(cyc[9], c4, r1);
         if (flipLane >= 0) {
-            const uint32_t x = __shfl(s, flipLane);
-            const bool qx = __shfl((int)qpos, flipLane) != 0;
+            const uint32_t x = (uint32_t)__builtin_amdgcn_readlane((int)s, flipLane);
+            const bool qx = __builtin_amdgcn_readlane((int)qpos, flipLane) != 0;
             const int nFl = kMultiCap ? uni(__popcll(flipMask)) : 1;
             nFlips += nFl;
             /* every flipped lane toggles its own site's bit (a site flipped
@@ -1147,7 +830,7 @@ __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y
                 const uint8_t *row = a.J8 + (long long)x * a.ld8;
                 waveSync();
                 ldsWait(); /* this wave's reads of `stage` and the scale are done */
-                dmaRunx4(row + lane * 16, stageL, a.ld8 / (kWave * 16));
+                dmaRunx4(row, stageL, a.ld8 / (kWave * 16));
                 if (lane == 0)
                     dmaDword<false>(a.rowScale + x, scaleL);
                 afterGroup += rowOps;
@@ -1176,7 +859,7 @@ __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y
                     issueMask &= issueMask - 1;
                     const uint32_t xr = (uint32_t)__builtin_amdgcn_readlane((int)s, fl);
                     const real *row = a.J + (long long)xr * Np;
-                    dmaRunx4(reinterpret_cast<const unsigned char *>(row + lane * 4), stageBufL(issueBuf), rowOps);
+                    dmaRunx4(reinterpret_cast<const unsigned char *>(row), stageBufL(issueBuf), rowOps);
                     afterGroup += rowOps;
                     ++issued;
                     issueBuf = (issueBuf + 1 == nBufs) ? 0 : issueBuf + 1;
@@ -1240,13 +923,7 @@ __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y
                 const real *row = a.J + (long long)x * Np;
                 waveSync();
                 ldsWait(); /* this wave's reads of `stage` are done */
-                uint32_t dst = stageL;
-                if constexpr (kHelp) {
-                    /* the other buffer than the one the helper may be reading */
-                    curStage ^= 1;
-                    dst = stageBufL(curStage);
-                }
-                dmaRunx4(reinterpret_cast<const unsigned char *>(row + lane * 4), dst, rowOps);
+                dmaRunx4(reinterpret_cast<const unsigned char *>(row), stageL, rowOps);
                 afterGroup += rowOps;
                 rowPending = true;
             } else if constexpr (!PLAIN) {
@@ -1295,11 +972,6 @@ __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y
 
     /* nothing may land in this region after the wave leaves it */
     vmWaitImm<0>();
-    if constexpr (kHelp) {
-        if (helpBusy)
-            while (helpLoad(ctl) != kHelpIdle)
-                ;
-    }
     if constexpr (kMultiCap) {
         if (nPend > 0 && !aborted) {
             applyPendingRows();
@@ -1326,8 +998,6 @@ __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y
             if (b + lane < Nw)
                 a.Qbits[(long long)y * Nw + b + lane] = Qb[b + lane];
     }
-    if constexpr (kHelp)
-        helpStore(ctl, kHelpExit);
     if (lane == 0 && a.counters) {
         atomicAdd(&a.counters[0], (unsigned long long)nFlips);
         atomicAdd(&a.counters[1], (unsigned long long)nBatches);
@@ -1339,7 +1009,7 @@ __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y
     }
 }
 
-template <class real, int MODE, bool MULTI = false, bool HELPER = false>
+template <class real, int MODE, bool MULTI = false>
 __global__ __launch_bounds__(kMaxSlicesPerBlock *kWave) void denseSweepKernel(SweepArgs<real> a, int slicesPerBlock,
                                                                                 int xcdRemap) {
     extern __shared__ __align__(16) unsigned char lds[];
@@ -1352,20 +1022,15 @@ __global__ __launch_bounds__(kMaxSlicesPerBlock *kWave) void denseSweepKernel(Sw
         int per = gridDim.x / 8;
         b = (blockIdx.x % 8) * per + blockIdx.x / 8;
     }
-    /* HELPER: one slice per block, wave 0 sweeps it and wave 1 applies rows */
-    const int y = HELPER ? b : b * slicesPerBlock + w;
+    const int y = b * slicesPerBlock + w;
 
     /* LDS carve-up: exp table, h, then one region per slice */
     uint64_t *expTab = reinterpret_cast<uint64_t *>(lds);
     real *hS = reinterpret_cast<real *>(lds + kExpTabBytes);
-    const size_t waveBytes = sweepWaveBytes<real, MODE>(a.Np, a.ld8, MULTI ? a.multiBufs : 0, HELPER);
-    unsigned char *p = lds + kExpTabBytes + (size_t)a.Np * sizeof(real) + waveBytes * (HELPER ? 0 : w);
+    const size_t waveBytes = sweepWaveBytes<real, MODE>(a.Np, a.ld8, MULTI ? a.multiBufs : 0);
+    unsigned char *p = lds + kExpTabBytes + (size_t)a.Np * sizeof(real) + waveBytes * w;
     if (threadIdx.x < 32)
         expTab[threadIdx.x] = sq_exp2_tab32[threadIdx.x];
-    if constexpr (HELPER) {
-        if (threadIdx.x == 0)
-            *helperCtl(a, p) = kHelpIdle;
-    }
     {
         /* h by DMA, the block's waves taking 1 KiB pieces in turn (h holds Np
          * reals, a multiple of 1 KiB) */
@@ -1379,13 +1044,7 @@ __global__ __launch_bounds__(kMaxSlicesPerBlock *kWave) void denseSweepKernel(Sw
     __syncthreads();
     if (y >= a.m)
         return;
-    if constexpr (HELPER) {
-        if (w == 1) {
-            helperLoop<real>(a, p);
-            return;
-        }
-    }
-    sweepSlice<real, MODE, MULTI, HELPER>(a, y, expTab, hS, p);
+    sweepSlice<real, MODE, MULTI>(a, y, expTab, hS, p);
 }
 
 /* Many instances in one persistent launch: every wave takes (instance,
@@ -1459,14 +1118,13 @@ void fp8DecodeTable(float out[256]) {
 }
 
 namespace {
-size_t waveBytesFor(int Np, size_t realSize, bool plain, int fieldFormat, int ld8, int multiBufs = 0,
-                    bool helper = false) {
+size_t waveBytesFor(int Np, size_t realSize, bool plain, int fieldFormat, int ld8, int multiBufs = 0) {
     if (realSize == 8)
         return plain ? sweepWaveBytes<double, kModePlain>(Np, ld8) : sweepWaveBytes<double, kModeLocal>(Np, ld8);
     if (plain)
         return sweepWaveBytes<float, kModePlain>(Np, ld8);
     return fieldFormat == fieldFP8 ? sweepWaveBytes<float, kModeFP8>(Np, ld8)
-                                   : sweepWaveBytes<float, kModeLocal>(Np, ld8, multiBufs, helper);
+                                   : sweepWaveBytes<float, kModeLocal>(Np, ld8, multiBufs);
 }
 
 template <class real>
@@ -1481,15 +1139,9 @@ void *batchKernelFor(bool plain, int fieldFormat) {
 }  // namespace
 
 size_t denseSweepLdsBytes(int Np, int slicesPerBlock, size_t realSize, bool plain, int fieldFormat, int ld8,
-                          int multiBufs, bool helper) {
+                          int multiBufs) {
     return kExpTabBytes + (size_t)Np * realSize +
-           waveBytesFor(Np, realSize, plain, fieldFormat, ld8, multiBufs, helper) * slicesPerBlock;
-}
-
-bool denseSweepHelperFits(int Np, int slicesPerBlock, size_t realSize, bool plain, int fieldFormat,
-                          size_t maxLds) {
-    return realSize == 4 && !plain && fieldFormat != fieldFP8 && slicesPerBlock == 1 &&
-           denseSweepLdsBytes(Np, 1, realSize, plain, fieldFormat, 0, 0, true) <= maxLds;
+           waveBytesFor(Np, realSize, plain, fieldFormat, ld8, multiBufs) * slicesPerBlock;
 }
 
 int denseSweepMultiBufs(int Np, int slicesPerBlock, size_t realSize, bool plain, int fieldFormat, size_t maxLds) {
@@ -1573,6 +1225,15 @@ static bool fitsAtOnce(const void *fn, int threads, size_t lds, int nBlocks, int
  * hold CUs finish, so the dispatched blocks all become resident.  If they
  * cannot (another process's spinning kernels), the spin limit turns the wait
  * into an error. */
+void launchSweep(void *kernel, int nBlocks, int threads, size_t lds, void **kargs, bool allowDirect, int numCUs,
+                 hipStream_t stream) {
+    HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    if (allowDirect && fitsAtOnce(kernel, threads, lds, nBlocks, numCUs))
+        HIP_CHECK(hipLaunchKernel(kernel, dim3(nBlocks), dim3(threads), kargs, (unsigned)lds, stream));
+    else
+        HIP_CHECK(hipLaunchCooperativeKernel(kernel, dim3(nBlocks), dim3(threads), kargs, (unsigned)lds, stream));
+}
+
 template <class real>
 void denseSweep(const SweepArgs<real> &args, bool plain, int fieldFormat, int slicesPerBlock, bool allowDirect,
                 int numCUs, hipStream_t stream) {
@@ -1582,15 +1243,9 @@ void denseSweep(const SweepArgs<real> &args, bool plain, int fieldFormat, int sl
     const bool fp8 = !plain && fieldFormat == fieldFP8;
     SQ_THROW_IF(fp8 && (sizeof(real) != 4 || !args.J8 || !args.rowScale || args.ld8 < args.Np || args.ld8 % 1024),
                 "fp8 sweep: needs a float solver and e4m3 rows with a 1 KiB-multiple stride");
-    /* the helper-wave kernel: float local-field form, single-flip batches,
-     * one slice per block */
-    const bool helper =
-        args.helperWave && sizeof(real) == 4 && !plain && !fp8 && args.multiBufs < 2 && slicesPerBlock == 1;
-    SQ_THROW_IF(args.helperWave && !helper && sizeof(real) == 4 && !plain && !fp8 && args.multiBufs < 2,
-                "helper-wave sweep: needs one slice per block");
     int nBlocks = divru(args.m, slicesPerBlock);
     size_t lds = denseSweepLdsBytes(args.Np, slicesPerBlock, sizeof(real), plain, fieldFormat, args.ld8,
-                                    args.multiBufs, helper);
+                                    args.multiBufs);
     int xcdRemap = (nBlocks % 8 == 0 && nBlocks >= 16) ? 1 : 0;
 
     void *fn = plain ? (void *)denseSweepKernel<real, kModePlain> : (void *)denseSweepKernel<real, kModeLocal>;
@@ -1599,17 +1254,10 @@ void denseSweep(const SweepArgs<real> &args, bool plain, int fieldFormat, int sl
             fn = (void *)denseSweepKernel<real, kModeFP8>;
         else if (!plain && args.multiBufs >= 2)
             fn = (void *)denseSweepKernel<real, kModeLocal, true>;
-        else if (helper)
-            fn = (void *)denseSweepKernel<real, kModeLocal, false, true>;
     }
-    const int threads = helper ? 2 * kWave : slicesPerBlock * kWave;
-    HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     SweepArgs<real> a = args;
     void *kargs[] = {(void *)&a, (void *)&slicesPerBlock, (void *)&xcdRemap};
-    if (allowDirect && fitsAtOnce(fn, threads, lds, nBlocks, numCUs))
-        HIP_CHECK(hipLaunchKernel(fn, dim3(nBlocks), dim3(threads), kargs, (unsigned)lds, stream));
-    else
-        HIP_CHECK(hipLaunchCooperativeKernel(fn, dim3(nBlocks), dim3(threads), kargs, (unsigned)lds, stream));
+    launchSweep(fn, nBlocks, slicesPerBlock * kWave, lds, kargs, allowDirect, numCUs, stream);
 }
 
 template void denseSweep<float>(const SweepArgs<float> &, bool, int, int, bool, int, hipStream_t);

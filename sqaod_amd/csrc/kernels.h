@@ -280,8 +280,8 @@ struct SweepArgs {
                              * flips (>= 2), 0: every batch ends at its first flip */
     int multiMinCand;       /* with multiBufs >= 2: accepting lanes of a batch that make the next batch
                              * commit all its flips */
-    int helperWave;         /* float local-field form, single-flip batches, one slice per block: a second
-                             * wave per slice applies the deferred J rows to the fields */
+    uint32_t *P;            /* team sweep: m x ldP published words, 16 decisions each */
+    int ldP;
 };
 
 /* multi_flip: "off", "auto" (the default: multi-flip batches in the first
@@ -301,14 +301,27 @@ template <class real>
 void denseSweep(const SweepArgs<real> &args, bool plain, int fieldFormat, int slicesPerBlock, bool allowDirect,
                 int numCUs, hipStream_t stream);
 
+/* Launches a sweep kernel whose blocks wait on each other: directly where
+ * allowDirect and all of them fit on the device at once, else cooperatively. */
+void launchSweep(void *kernel, int nBlocks, int threads, size_t lds, void **kargs, bool allowDirect, int numCUs,
+                 hipStream_t stream);
+
+/* The local-field sweep (float: rows of args.J; double) by a team of four waves
+ * per slice, each batch ending at its first flip (dense_sweep_team.hip).
+ * args.P: m rows of args.ldP >= teamWordStride(N) words, cleared before the first
+ * sweep and every kTeamTagPeriod sweeps (args.tag % kTeamTagPeriod == 0). */
+constexpr uint32_t kTeamTagPeriod = 2047;
+int teamWordStride(int N);
+/* Slices per block (asked: 0 to choose), 0 where the sweep does not fit. */
+int denseSweepTeamSlices(int N, int Np, int m, size_t realSize, int asked, int numCUs, size_t maxLds);
+template <class real>
+void denseSweepTeam(const SweepArgs<real> &args, int slicesPerBlock, size_t maxLds, bool allowDirect, int numCUs,
+                    hipStream_t stream);
+
 /* Bytes of LDS one block of the local-field sweep needs (ld8: the fp8 row
  * stride, used when fieldFormat == fieldFP8). */
 size_t denseSweepLdsBytes(int Np, int slicesPerBlock, size_t realSize, bool plain, int fieldFormat = fieldF32,
-                          int ld8 = 0, int multiBufs = 0, bool helper = false);
-/* Whether the helper-wave sweep (SweepArgs::helperWave) applies and fits in
- * maxLds bytes per block. */
-bool denseSweepHelperFits(int Np, int slicesPerBlock, size_t realSize, bool plain, int fieldFormat,
-                          size_t maxLds);
+                          int ld8 = 0, int multiBufs = 0);
 /* Row stage buffers for multi-flip batches that fit beside S slices' regions
  * in maxLds bytes (0: none; at most 4, and (buffers - 1) rows of DMA ops within
  * the 63 outstanding memory operations a wave can count). */

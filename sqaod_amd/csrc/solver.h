@@ -244,8 +244,8 @@ private:
     int multiFlipMode_ = kMultiFlipAuto;
     int multiFlipMin_ = kMultiFlipDefaultMin;
     int sweepsSinceSpinsSet_ = 0;
-    /* single-flip float local-field sweeps with one slice per block: a second
-     * wave per slice applies the deferred J rows (where LDS allows) */
+    /* single-flip local-field sweeps run four waves per slice (the team
+     * sweep, where LDS allows) */
     bool helperWave_ = true;
     int sysTraceCap_ = 0, sysTraceLen_ = 0;
     long long sysTraceSteps_ = 0;
@@ -282,6 +282,8 @@ private:
     DevBuf<int> d_rowExp_;
     int ld8_ = 0;
     DevBuf<uint32_t> d_Q_, d_X_, d_D_, d_words_;
+    DevBuf<uint32_t> d_P_; /* the team sweep's published words, m x ldP_ */
+    int ldP_ = 0;
     DevBuf<MTState> d_mt_;
     DevBuf<double> d_E_, d_partial_, d_spinDot_;
     /* energies: J as int8 digit planes for the integer MFMA, built once per J */

@@ -60,8 +60,9 @@ SQ_HD static inline double sq_u2d(uint64_t u) {
 #define SQ_EXPF_FUSED_POLY 1
 #endif
 
-/* tab: the 32-entry table above, or a copy of it (e.g. in GPU LDS). */
-SQ_HD static inline float sq_expf_tab(float x, const uint64_t *tab) {
+/* 2^(k/32) 2^(r/32) for a finite x of moderate size, before its one rounding to
+ * float.  tab: the 32-entry table above, or a copy of it (e.g. in GPU LDS). */
+SQ_HD static inline double sq_exp_double(float x, const uint64_t *tab) {
 #ifdef __clang__
 #pragma clang fp contract(off)
 #endif
@@ -72,11 +73,6 @@ SQ_HD static inline float sq_expf_tab(float x, const uint64_t *tab) {
     const double C1 = 0x1.ebfce50fac4f3p-3 / (32.0 * 32.0);
     const double C2 = 0x1.62e42ff0c52d6p-1 / 32.0;
 
-    /* The special inputs are selected after the main path instead of
-     * branching before it (a wave whose lanes straddle |x| = 88 would run
-     * both sides); the main path is evaluated for every input, with a finite
-     * table index, and its result is replaced for x < -103.97 (rounds to +0,
-     * also -inf), x > 88.72 (rounds to +inf, also +inf) and NaN (x + x). */
     double xd = (double)x;
 #if SQ_EXPF_FUSED_REDUCTION
     double kd = __builtin_fma(InvLn2N, xd, Shift);
@@ -103,8 +99,16 @@ SQ_HD static inline float sq_expf_tab(float x, const uint64_t *tab) {
     double y = C2 * r + 1.0;
     y = p * r2 + y;
 #endif
-    y = y * s;
-    float res = (float)y;
+    return y * s;
+}
+
+SQ_HD static inline float sq_expf_tab(float x, const uint64_t *tab) {
+    /* The special inputs are selected after the main path instead of
+     * branching before it (a wave whose lanes straddle |x| = 88 would run
+     * both sides); the main path is evaluated for every input, with a finite
+     * table index, and its result is replaced for x < -103.97 (rounds to +0,
+     * also -inf), x > 88.72 (rounds to +inf, also +inf) and NaN (x + x). */
+    float res = (float)sq_exp_double(x, tab);
     res = (x < -0x1.9fe368p6f) ? 0x1p-95f * 0x1p-95f : res;
     res = (x > 0x1.62e42ep6f) ? 0x1p97f * 0x1p97f : res;
     res = (x != x) ? x + x : res;
@@ -112,3 +116,42 @@ SQ_HD static inline float sq_expf_tab(float x, const uint64_t *tab) {
 }
 
 SQ_HD static inline float sq_expf(float x) { return sq_expf_tab(x, sq_exp2_tab32); }
+
+/* The least float x with sq_expf(x) > u, for a float u in [0, 1); NaN for
+ * u >= 1.  sq_expf is monotone on the floats below zero (checked for all of
+ * them by tests/test_expf_above_cpu.py), so for every float x
+ *   sq_expf(x) > u   <=>   x >= sq_exp_above(u)      (u < 1; x NaN: both false).
+ * A Newton step in double from a rough logarithm of the midpoint between u and
+ * the next float lands within a few floats of it; the loops, which test
+ * sq_expf itself, settle the rest. */
+SQ_HD static inline float sq_exp_above(float u, const uint64_t *tab) {
+#ifdef __clang__
+#pragma clang fp contract(off)
+#endif
+    union { uint32_t b; float f; } x, n;
+    if (!(u < 1.0f)) {
+        x.b = 0x7fc00000u;
+        return x.f;
+    }
+    if (!(u > 0.0f))
+        return -0x1.9fe368p6f; /* sq_expf is the least denormal here and 0 below */
+    n.b = sq_f2u(u) + 1u;
+    const double mid = 0.5 * ((double)u + (double)n.f);
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float x0 = __logf((float)mid);
+#else
+    const float x0 = __builtin_logf((float)mid);
+#endif
+    x.f = (float)((double)x0 + (mid - sq_exp_double(x0, tab)) * (double)(1.0f / (float)mid));
+    if (!(x.f < 0.0f))
+        x.b = 0x80000001u; /* the answer is below zero */
+    while (!(sq_expf_tab(x.f, tab) > u))
+        --x.b; /* negative: the next float up */
+    for (;;) {
+        n.b = x.b + 1u;
+        if (!(sq_expf_tab(n.f, tab) > u))
+            break;
+        x = n;
+    }
+    return x.f;
+}

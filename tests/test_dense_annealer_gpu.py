@@ -440,3 +440,38 @@ def test_helper_wave_near_the_lds_limit(oracle, rocm):
         an.anneal_one_step(G, BETA)
     assert np.array_equal(q_of(an), ora.get_q())
     assert np.array_equal(an.get_E(), ora.calculate_E())
+
+
+@pytest.mark.parametrize("N,m,spb,dtype,algo", [
+    (5, 2, 2, np.float32, "coloring"), (63, 5, 4, np.float64, "coloring"), (65, 3, 1, np.float32, "coloring"),
+    (255, 9, 3, np.float32, "coloring"), (257, 6, 2, np.float64, "coloring"), (1024, 4, 4, np.float32, "coloring"),
+    (1025, 4, 2, np.float32, "coloring"), (1025, 3, 1, np.float64, "coloring"), (200, 5, 4, np.float64, "sa_naive")])
+def test_team_sweep_bit_exact(oracle, rocm, N, m, spb, dtype, algo):
+    """The team sweep at the sizes where its rings (256 prepared attempts),
+    words of 16 decisions, chunks of 64 and tables by site (shared slots
+    resolved up to N = 1024) wrap or change, 1 to 4 slices per workgroup with
+    the ring of slices closing inside one or not, float and double: the serial
+    CPU annealer's spins and energies, bit for bit."""
+    W = dense_int_W(N, SEED_BASE + 7 * N + m)
+    ora, an = make_pair(oracle, rocm, W, m, seed=11 + N, algo=algo, dtype=dtype, multi_flip="off",
+                        slices_per_block=spb)
+    for G in (np.geomspace(20.0, 0.05, 30) if algo == "sa_naive" else schedule()[:160:5]):
+        beta = 0.0 if algo == "sa_naive" else BETA
+        ora.anneal_one_step(G, beta)
+        an.anneal_one_step(G, beta)
+        assert np.array_equal(q_of(an), ora.get_q())
+    assert np.array_equal(an.get_E(), ora.calculate_E())
+
+
+def test_team_sweep_past_its_tag_period(oracle, rocm):
+    """More sweeps than the published words have tags (2047)."""
+    N, m = 24, 4
+    W = dense_int_W(N, SEED_BASE + 3)
+    ora, an = make_pair(oracle, rocm, W, m, seed=5, multi_flip="off")
+    for k in range(2150):
+        G = 3.0 if k % 50 else 0.5
+        ora.anneal_one_step(G, 1.0)
+        an.anneal_one_step(G, 1.0)
+        if k > 2030 and k % 20 == 0:
+            assert np.array_equal(q_of(an), ora.get_q()), k
+    assert np.array_equal(q_of(an), ora.get_q())

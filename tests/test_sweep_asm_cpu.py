@@ -42,6 +42,25 @@ def sweep_asm(tmp_path_factory):
     return _device_asm(tmp_path_factory, "dense_sweep.hip")
 
 
+@pytest.fixture(scope="module")
+def team_asm(tmp_path_factory):
+    return _device_asm(tmp_path_factory, "dense_sweep_team.hip")
+
+
+def test_team_sweep_uses_no_scratch_and_no_m0(team_asm):
+    """The same for the team sweep's kernels (dense_sweep_team.hip)."""
+    parts = re.split(r";;#ASM(?:START|END)", team_asm)  # inside and outside inline assembly in turn
+    for text in parts[0::2]:
+        for line in text.splitlines():
+            assert line.strip().startswith(";") or not re.search(r"\bm0\b", line), line
+    assert sum(len(re.findall(r"s_mov_b32\s+m0,", text)) for text in parts[1::2]) > 0
+    names = re.findall(r"\.name:\s+(\S*denseSweepTeam\S*)\n(.*?)(?=\n\s+- \.|\Z)", team_asm, flags=re.S)
+    assert len(names) == 2
+    for name, meta in names:
+        assert re.search(r"\.private_segment_fixed_size:\s+0\b", meta), name
+        assert re.search(r"\.vgpr_spill_count:\s+0\b", meta), name
+
+
 @pytest.mark.parametrize("src, pattern", [("dense_sweep.hip", "denseSweep"),
                                           ("dense_field_mfma.hip", "fieldRefresh")])
 def test_kernels_use_no_scratch(tmp_path_factory, sweep_asm, src, pattern):
