@@ -86,11 +86,11 @@ int sqaod_rocm_dg_annealer_get_problem_size(sqaod_rocm_dg_annealer *a, int *N);
  * sweeps commit every flip of a 64-attempt batch in order, instead of ending
  * the batch at its first flip, after a batch with at least 4 (or the given
  * number of) accepting lanes; "auto" does so in the first 3 sweeps after the
- * spins were set, when most attempts are accepted; the results are the same
- * in every mode),
- * "helper_wave" ("on" | "off": single-flip float local-field sweeps with one
- * slice per workgroup run a second wave per slice that applies the deferred
- * J rows to the fields; the results are the same either way),
+ * spins were set, when most attempts are accepted, where helper_wave does not
+ * apply; the results are the same in every mode),
+ * "helper_wave" ("on" | "off": single-flip local-field sweeps run by a team of
+ * four waves per slice where they fit in LDS; the results are the same either
+ * way),
  * "slices_per_block" (int, 0 = auto), "sweep_launch" ("auto" | "cooperative"),
  * "refresh_interval" (int, steps between
  * field recomputes; 0 = only after the spins were set), "refresh_engine"

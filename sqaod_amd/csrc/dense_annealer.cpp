@@ -378,8 +378,9 @@ void DenseGraphAnnealer<real>::setPreference(const std::string &name, const std:
     } else if (name == "multi_flip") {
         /* float local-field sweeps: "off" (every batch ends at its first
          * flip), "auto" (multi-flip batches in the first sweeps after the
-         * spins were set), "on" (in every sweep), or a number 2..64: "on"
-         * with that threshold of accepting lanes */
+         * spins were set, where the team sweep does not run), "on" (in every
+         * sweep), or a number 2..64: "on" with that threshold of accepting
+         * lanes */
         if (value == "on" || value == "true" || value == "True") {
             multiFlipMode_ = kMultiFlipOn;
             multiFlipMin_ = kMultiFlipDefaultMin;
@@ -900,11 +901,19 @@ void DenseGraphAnnealer<real>::annealOneStep(real G, real beta) {
     SQ_THROW_IF(denseSweepLdsBytes(Np_, S, sizeof(real), plainSweep_, fieldFormat_, ld8_) > dev_->maxLdsPerBlock(),
                 "N=%d too large for the LDS-resident sweep (%zu bytes needed per block)", N_,
                 denseSweepLdsBytes(Np_, S, sizeof(real), plainSweep_, fieldFormat_, ld8_));
-    /* multi-flip batches where LDS allows (float local-field sweeps).  The
-     * fp8 form's run the float kernel on the float copy of J' (a.J): its row
-     * updates add the same values, -+2 J'[x][s], exactly. */
-    const bool multi = multiFlipMode_ == kMultiFlipOn ||
-                       (multiFlipMode_ == kMultiFlipAuto && sweepsSinceSpinsSet_ < kMultiFlipAutoSweeps);
+    /* the team sweep where it fits; the fp8 form's runs on the float copy of J'
+     * (a.J): its row updates add the same values, -+2 J'[x][s], exactly */
+    int teamS = 0;
+    if (helperWave_ && !plainSweep_)
+        teamS = denseSweepTeamSlices(N_, Np_, m_, sizeof(real), slicesPerBlock_, dev_->numCUs(), dev_->maxLdsPerBlock());
+    /* multi-flip batches where LDS allows (float local-field sweeps; the fp8
+     * form's on the float copy of J' as well).  "auto" takes them in the first
+     * sweeps only beside the one-wave kernel: the team sweep is faster there but
+     * for the very first sweep of some sizes (us, sweeps 0-2, multi-flip / team:
+     * N=4096, m=256 1980 1260 969 / 1897 1019 677; N=2048, m=128 851 549 428 /
+     * 970 533 350; N=128, m=32 136 109 108 / 71 47 33) */
+    const bool multi = multiFlipMode_ == kMultiFlipOn || (multiFlipMode_ == kMultiFlipAuto && teamS == 0 &&
+                                                          sweepsSinceSpinsSet_ < kMultiFlipAutoSweeps);
     int sweepFormat = fieldFormat_;
     a.multiMinCand = multiFlipMin_;
     a.multiBufs = 0;
@@ -918,12 +927,7 @@ void DenseGraphAnnealer<real>::annealOneStep(real G, real beta) {
     const bool direct = !coopLaunch_ && dev_->soleSweeper();
     if (profile_)
         phaseBegin(2, pe);
-    /* the team sweep where it fits; the fp8 form's runs on the float copy of J'
-     * (a.J) as well */
-    int teamS = 0;
-    if (helperWave_ && !plainSweep_ && a.multiBufs < 2)
-        teamS = denseSweepTeamSlices(N_, Np_, m_, sizeof(real), slicesPerBlock_, dev_->numCUs(), dev_->maxLdsPerBlock());
-    if (teamS > 0) {
+    if (teamS > 0 && a.multiBufs < 2) {
         if (a.tag % kTeamTagPeriod == 0) /* its words' tags start over */
             HIP_CHECK(hipMemsetAsync(d_P_.ptr, 0, d_P_.bytes(), dev_->stream()));
         denseSweepTeam<real>(a, teamS, dev_->maxLdsPerBlock(), direct, dev_->numCUs(), dev_->stream());

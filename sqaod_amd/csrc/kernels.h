@@ -285,8 +285,8 @@ struct SweepArgs {
 };
 
 /* multi_flip: "off", "auto" (the default: multi-flip batches in the first
- * kMultiFlipAutoSweeps sweeps after the spins were set, when most attempts
- * are accepted), "on" (every sweep), each with the threshold "on" stands
+ * kMultiFlipAutoSweeps sweeps after the spins were set, when most attempts are
+ * accepted, where the team sweep does not run), "on" (every sweep), each with the threshold "on" stands
  * for unless a number is given. */
 enum { kMultiFlipOff = 0, kMultiFlipAuto = 1, kMultiFlipOn = 2 };
 constexpr int kMultiFlipDefaultMin = 4;
