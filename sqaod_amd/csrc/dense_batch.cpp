@@ -215,7 +215,7 @@ void GroupedDenseStepper::run(Device &dev, const std::vector<DenseGraphAnnealer<
             if (a.refreshDue()) {
                 FieldGemmJob j = a.takeFieldGemmJob();
                 gs.push_back(gBlocks);
-                gBlocks += fieldGemmJobBlocks(j, o.fieldFormat);
+                gBlocks += fieldGemmJobBlocks(j);
                 gj.push_back(j);
             }
             AttemptStreamJob s = a.takeAttemptStreamJob();

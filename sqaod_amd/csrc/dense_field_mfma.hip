@@ -23,17 +23,26 @@
  * load of a wave is a single fully coalesced 1 KiB request and a block
  * streams its columns' k-range front to back.
  *
- * Work split: one block of 4 waves owns 16 output columns and all slice rows
- * of a pass (up to 256: sixteen 16 x 16 accumulator tiles per wave).  The
- * k-range is split over the 4 waves in super-blocks of kDepth k-blocks
- * (interleaved), each wave double-buffers its operand loads, and the four
- * partial sums are added in a fixed order through LDS, so results are
- * deterministic.  Each block starts its k-range at a different super-block,
- * so concurrently running blocks read different address ranges.
+ * Work split: one block of 4 waves owns 16 output columns and T tiles of 16
+ * slice rows.  The k-range is split over the 4 waves in super-blocks of kDepth
+ * k-blocks (interleaved), each wave double-buffers its operand loads, and the
+ * four partial sums are added in a fixed order through LDS, so results are
+ * deterministic and do not depend on T.  Each column block starts its k-range at
+ * a different super-block, so concurrently running blocks read different address
+ * ranges; the row groups of a column block run on one XCD, next to each other,
+ * and find its fragments in that XCD's L2.
  *
- * Spins: lane L loads the packed spin words of slice row y0 + 64 r + L for a
- * whole super-block (one 16-byte load per row group); the A fragment of tile
- * t is then fetched from the owning lane with ds_bpermute (__shfl).
+ * What bounds it is the chain of a wave's round trips (operands, the spin table
+ * in LDS), so T is the largest that leaves two blocks to each CU (rowTilesFor).
+ * With T = 16 throughout, i.e. each column block in one block, whose spin words
+ * went through a lane shuffle, the refresh of N=4096, m=256 (bf16x2) took
+ * 35.2 us, that of N=1200, m=300 (fp32) 24.3 us and a half-step of the bipartite
+ * 1024 + 1024, m=64 8.3 us; now 29.7, 8.5 and 4.1 us.  A large bf16 product
+ * would take 14 us for the first, and so would reading its fragments once.
+ *
+ * Spins: lane L loads the packed spin words of row L % 16 of each tile for a
+ * whole super-block (16 bytes); a byte of them picks 8 spins as bf16 +-1 from a
+ * table in LDS.
  *
  * The k-blocks past the valid length read zero padding (rows of B are padded
  * to K with zeros, the fragment copy is zero for columns past B's rows, and
@@ -52,8 +61,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kWave = 64;
-constexpr int kTiles = 16;        /* 16-row accumulator tiles per wave: 256 slice rows per pass */
-constexpr int kRowsPerPass = kTiles * 16;
+constexpr int kGroupedTiles = 4;  /* row tiles per block of a grouped launch */
 constexpr int kSplitK = 4;        /* waves per block, each a share of the k-range */
 constexpr int kDepth = 4;         /* k-blocks per super-block (the double-buffered unit) */
 constexpr int kBlockThreads = kSplitK * kWave;
@@ -68,178 +76,122 @@ __device__ __forceinline__ bf16x8 spinsBF16(uint32_t bits) {
     return __builtin_bit_cast(bf16x8, v);
 }
 
+/* The partial tiles: [w][4 t + r][lane] holds wave w's acc[t][r], i.e. row
+ * 16 t + 4 (lane / 16) + r, column lane % 16. */
+template <int T>
+using RedTile = float[T * 4][kWave];
+
 /* Fixed-order sum of the kSplitK partial tiles in LDS and the store of the
- * pass's rows: red[w][4 t + r][lane] holds wave w's acc[t][r]; colScale (if
- * given) multiplies each column's sum. */
-__device__ __forceinline__ void reduceStore(float (*red)[kTiles * 4][kWave], int y0, int m, int cb, int ldF, float *F,
-                                            const float *colScale = nullptr) {
-    __syncthreads();
-#pragma unroll 4
-    for (int j = 0; j < kTiles * 4 * kWave / kBlockThreads; ++j) {
-        const int o = j * kBlockThreads + threadIdx.x;
-        const int tr = o / kWave, L = o % kWave;
-        const int y = y0 + 16 * (tr >> 2) + 4 * (L >> 4) + (tr & 3);
-        if (y < m) {
-            float s = red[0][tr][L];
+ * block's rows; colScale (if given) multiplies each column's sum. */
+template <int T>
+__device__ __forceinline__ void reduceStore(const f32x4 (&acc)[T], RedTile<T> *red, int y0, int m, int cb, int ldF,
+                                            float *F, const float *colScale = nullptr) {
+    const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
 #pragma unroll
-            for (int w = 1; w < kSplitK; ++w)
-                s += red[w][tr][L];
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            red[w][4 * t + r][lane] = acc[t][r];
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        /* wave w adds register w of each tile */
+        const int y = y0 + 16 * t + 4 * (lane >> 4) + w, col = cb * 16 + (lane & 15);
+        if (y < m) {
+            float s = red[0][4 * t + w][lane];
+#pragma unroll
+            for (int p = 1; p < kSplitK; ++p)
+                s += red[p][4 * t + w][lane];
             if (colScale)
-                s *= colScale[cb * 16 + (L & 15)];
-            F[(long long)y * ldF + cb * 16 + (L & 15)] = s;
+                s *= colScale[col];
+            F[(long long)y * ldF + col] = s;
         }
     }
-    __syncthreads();
 }
-
-typedef float RedTile[kTiles * 4][kWave];
-
-/* In a grouped launch the bf16 forms split the waves of a workgroup over
- * columns instead of the k-range when the k-range is at most kColSplitMaxK:
- * many small GEMMs then fill the device with a quarter of the workgroups and
- * no LDS reduction, in the same summation order (refreshBF16Block).  A GEMM
- * alone keeps the k-split, which fills the device better. */
-constexpr int kColSplitMaxK = 2048;
-__host__ __device__ inline bool bf16ColSplit(int K) { return K <= kColSplitMaxK; }
 
 /* frag: [column blocks][K/32 k-blocks][PLANES][64 lanes] x 16 B (PLANES bf16
  * planes whose sum is B: hi + lo for the bf16x2 form, hi + mid + lo -- exactly
- * B -- for the fp32 form); the block writes columns [16 cb, 16 cb + 16) of F
- * (row stride ldF).  lut: byte -> 8 spins as bf16 +-1, filled by the caller. */
-template <int PLANES, bool colSplit = false>
+ * B -- for the fp32 form); the block writes columns [16 cb, 16 cb + 16) of rows
+ * [y0, y0 + 16 T) of F (row stride ldF).  lut: byte -> 8 spins as bf16 +-1. */
+template <int PLANES, int T>
 __device__ __forceinline__ void refreshBF16Block(const uint4 *frag, const uint32_t *Qbits, int K, int m, int Nw,
-                                                 int ldF, float *F, int cbBlock, RedTile *red, const uint4 *lut) {
+                                                 int ldF, float *F, int cb, int y0, RedTile<T> *red,
+                                                 const uint4 *lut) {
     const int lane = threadIdx.x % kWave;
     const int w = threadIdx.x / kWave;
     const int c = lane & 15, g = lane >> 4;
     const int nK = K / 32;      /* k-blocks of 32; K is a multiple of 256 */
-    const int nS = nK / kDepth; /* super-blocks */
-    /* Without colSplit the four waves take the super-blocks l = w, w + 4, ...
-     * of column block cbBlock and their partial tiles are added in LDS in the
-     * order ((P0 + P1) + P2) + P3.  With colSplit each wave owns a column block
-     * of its own (block cbBlock covers column blocks 4 cbBlock .. 4 cbBlock + 3)
-     * and forms the same partials P0..P3 one after the other, adding them in
-     * the same order: the results are bit-identical, without the LDS
-     * reduction and with a quarter of the workgroups. */
-    const int cb = colSplit ? cbBlock * kSplitK + w : cbBlock;
-    const int nParts = colSplit ? kSplitK : 1;
+    const int nS = nK / kDepth; /* super-blocks: wave w takes w, w + 4, ... */
     const int sOff = (int)(((long long)cb * 3) % nS);
     const uint4 *fb = frag + (size_t)cb * nK * PLANES * kWave + lane;
-    for (int y0 = 0; y0 < m; y0 += kRowsPerPass) {
-        f32x4 acc[kTiles], total[kTiles];
-      for (int part = 0; part < nParts; ++part) {
-        const int lStart = colSplit ? part : w;
-        constexpr int lStride = kSplitK;
+    f32x4 acc[T];
 #pragma unroll
-        for (int t = 0; t < kTiles; ++t)
-            acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        uint4 bp[PLANES][2][kDepth], qw[2][kTiles / 4];
-        /* loads super-block l (logical index) into buffer buf; l < nS */
-        auto fetch = [&](int buf, int l) {
-            int s = l + sOff;
-            if (s >= nS)
-                s -= nS;
-            const int kb0 = s * kDepth;
+    for (int t = 0; t < T; ++t)
+        acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    uint4 bp[PLANES][2][kDepth], qw[2][T];
+    /* loads super-block l (logical index) into buffer buf; l < nS.  Rows past
+     * m read row m - 1; their sums are not stored. */
+    auto fetch = [&](int buf, int l) {
+        int s = l + sOff;
+        if (s >= nS)
+            s -= nS;
+        const int kb0 = s * kDepth;
 #pragma unroll
-            for (int d = 0; d < kDepth; ++d) {
-                const uint4 *p = fb + (size_t)(kb0 + d) * PLANES * kWave;
+        for (int d = 0; d < kDepth; ++d) {
+            const uint4 *p = fb + (size_t)(kb0 + d) * PLANES * kWave;
+#pragma unroll
+            for (int pl = 0; pl < PLANES; ++pl)
+                bp[pl][buf][d] = p[pl * kWave];
+        }
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const int y = y0 + 16 * t + c;
+            qw[buf][t] = *reinterpret_cast<const uint4 *>(Qbits + (size_t)(y < m ? y : m - 1) * Nw + kb0);
+        }
+    };
+    /* the A operands of a k-block are read from the table one k-block ahead of
+     * the MFMAs that use them */
+    auto gather = [&](int buf, int d, uint4 *av) {
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const uint4 q4 = qw[buf][t];
+            const uint32_t word = d == 0 ? q4.x : d == 1 ? q4.y : d == 2 ? q4.z : q4.w;
+            av[t] = lut[(word >> (8 * g)) & 0xffu];
+        }
+    };
+    auto compute = [&](int buf) {
+        uint4 av[2][T];
+        gather(buf, 0, av[0]);
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d) {
+            if (d + 1 < kDepth)
+                gather(buf, d + 1, av[(d + 1) & 1]);
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                if (y0 + 16 * t >= m) /* wave-uniform */
+                    continue;
 #pragma unroll
                 for (int pl = 0; pl < PLANES; ++pl)
-                    bp[pl][buf][d] = p[pl * kWave];
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        __builtin_bit_cast(bf16x8, av[d & 1][t]), __builtin_bit_cast(bf16x8, bp[pl][buf][d]), acc[t], 0,
+                        0, 0);
             }
-            /* words kb0 .. kb0+3 of row y0 + 64 r + lane (kb0 is a multiple of 4, Nw of 8);
-             * rows past m read row m - 1 and are zeroed, so every load is
-             * unconditional and the waits before compute count precisely */
-#pragma unroll
-            for (int r = 0; r < kTiles / 4; ++r) {
-                const int y = y0 + 64 * r + lane;
-                const uint4 v = *reinterpret_cast<const uint4 *>(Qbits + (size_t)(y < m ? y : m - 1) * Nw + kb0);
-                qw[buf][r] = (y < m) ? v : uint4{0u, 0u, 0u, 0u};
-            }
-        };
-        /* A operands of four tiles are gathered (lane shuffle, then table
-         * read) one group ahead of the MFMAs that use them, so a group's LDS
-         * round trips run under the previous group's MFMAs; a pass with all
-         * 16 tiles in range has no per-tile branch at all */
-        const bool fullPass = y0 + kRowsPerPass <= m;
-        constexpr int kGroups = kTiles / 4;
-        auto groupLive = [&](int t0) { return fullPass || y0 + 16 * t0 < m; }; /* wave-uniform */
-        auto gather = [&](int buf, int step, uint4 a4[4]) {
-            const int d = step / kGroups, t0 = (step % kGroups) * 4;
-            if (!groupLive(t0))
-                return;
-            const uint4 q4 = qw[buf][t0 >> 2];
-            const uint32_t qd = d == 0 ? q4.x : d == 1 ? q4.y : d == 2 ? q4.z : q4.w;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const uint32_t word = (uint32_t)__shfl((int)qd, 16 * u + c, kWave);
-                a4[u] = lut[(word >> (8 * g)) & 0xffu];
-            }
-        };
-        auto compute = [&](int buf) {
-            uint4 a4[2][4];
-            gather(buf, 0, a4[0]);
-#pragma unroll
-            for (int step = 0; step < kDepth * kGroups; ++step) {
-                if (step + 1 < kDepth * kGroups)
-                    gather(buf, step + 1, a4[(step + 1) & 1]);
-                const int d = step / kGroups, t0 = (step % kGroups) * 4;
-                if (!groupLive(t0))
-                    continue;
-
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int t = t0 + u;
-                    if (fullPass || y0 + 16 * t < m) {
-                        const bf16x8 av = __builtin_bit_cast(bf16x8, a4[step & 1][u]);
-#pragma unroll
-                        for (int pl = 0; pl < PLANES; ++pl)
-                            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                                av, __builtin_bit_cast(bf16x8, bp[pl][buf][d]), acc[t], 0, 0, 0);
-                    }
-                }
-            }
-        };
-        /* buffers alternate with constant indices (no dynamic register indexing) */
-        for (int l = lStart; l < nS; l += 2 * lStride) {
-            if (l == lStart)
-                fetch(0, l);
-            if (l + lStride < nS)
-                fetch(1, l + lStride);
-            compute(0);
-            if (l + lStride >= nS)
-                break;
-            if (l + 2 * lStride < nS)
-                fetch(0, l + 2 * lStride);
-            compute(1);
         }
-        if (colSplit) {
-#pragma unroll
-            for (int t = 0; t < kTiles; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    total[t][r] = part == 0 ? acc[t][r] : total[t][r] + acc[t][r];
-        }
-      }
-        if (colSplit) {
-            /* tile t, register r: row y0 + 16 t + 4 (lane / 16) + r, column 16 cb + lane % 16 */
-#pragma unroll
-            for (int t = 0; t < kTiles; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int y = y0 + 16 * t + 4 * g + r;
-                    if (y < m)
-                        F[(long long)y * ldF + cb * 16 + c] = total[t][r];
-                }
-            continue;
-        }
-#pragma unroll
-        for (int t = 0; t < kTiles; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                red[w][4 * t + r][lane] = acc[t][r];
-        reduceStore(red, y0, m, cb, ldF, F);
+    };
+    /* buffers alternate with constant indices (no dynamic register indexing) */
+    for (int l = w; l < nS; l += 2 * kSplitK) {
+        if (l == w)
+            fetch(0, l);
+        if (l + kSplitK < nS)
+            fetch(1, l + kSplitK);
+        compute(0);
+        if (l + kSplitK >= nS)
+            break;
+        if (l + 2 * kSplitK < nS)
+            fetch(0, l + 2 * kSplitK);
+        compute(1);
     }
+    reduceStore<T>(acc, red, y0, m, cb, ldF, F);
 }
 
 __device__ __forceinline__ void fillLutBF16(uint4 *lut) {
@@ -248,22 +200,45 @@ __device__ __forceinline__ void fillLutBF16(uint4 *lut) {
     __syncthreads();
 }
 
-__global__ __launch_bounds__(kBlockThreads) void fieldRefreshBF16x2Kernel(const uint4 *frag, const uint32_t *Qbits,
-                                                                          int K, int m, int Nw, int ldF, float *F) {
-    __shared__ float red[kSplitK][kTiles * 4][kWave]; /* 64 KiB */
-    __shared__ uint4 lut[256];                        /* 4 KiB */
-    fillLutBF16(lut);
-    refreshBF16Block<2>(frag, Qbits, K, m, Nw, ldF, F, blockIdx.x, red, lut);
+/* Column block and first row of a block: the row groups of one column block are
+ * 8 apart, i.e. on one XCD one after the other (nColBlocks is a multiple of 8,
+ * or the tail of it keeps the plain order). */
+__device__ __forceinline__ void blockTile(int block, int nColBlocks, int nGroups, int rows, int &cb, int &y0) {
+    const int whole = nColBlocks / 8 * 8 * nGroups;
+    int group;
+    if (block < whole) {
+        const int i = block / 8;
+        cb = i / nGroups * 8 + block % 8;
+        group = i % nGroups;
+    } else {
+        cb = nColBlocks / 8 * 8 + (block - whole) / nGroups;
+        group = (block - whole) % nGroups;
+    }
+    y0 = group * rows;
 }
 
-__global__ __launch_bounds__(kBlockThreads) void fieldRefreshBF16x3Kernel(const uint4 *frag, const uint32_t *Qbits,
-                                                                          int K, int m, int Nw, int ldF, float *F) {
-    __shared__ float red[kSplitK][kTiles * 4][kWave]; /* 64 KiB */
-    __shared__ uint4 lut[256];                        /* 4 KiB */
+template <int PLANES, int T>
+__global__ __launch_bounds__(kBlockThreads) void fieldRefreshBF16Kernel(const uint4 *frag, const uint32_t *Qbits,
+                                                                        int nColBlocks, int nGroups, int K, int m,
+                                                                        int Nw, int ldF, float *F) {
+    __shared__ RedTile<T> red[kSplitK];
+    __shared__ uint4 lut[256]; /* 4 KiB */
+    int cb, y0;
+    blockTile(blockIdx.x, nColBlocks, nGroups, 16 * T, cb, y0);
     fillLutBF16(lut);
-    refreshBF16Block<3>(frag, Qbits, K, m, Nw, ldF, F, blockIdx.x, red, lut);
+    refreshBF16Block<PLANES, T>(frag, Qbits, K, m, Nw, ldF, F, cb, y0, red, lut);
 }
 
+/* Row tiles per block: the largest of 1, 2, 4 that leaves 512 blocks, two to each
+ * of the 256 CUs.  (Eight take 292 registers, one wave to a SIMD: N=4096, m=256
+ * bf16x2 33.1 us against 29.7 us with four.) */
+int rowTilesFor(int nColBlocks, int m) {
+    const int tiles = divru(m, 16);
+    for (int t = 4; t > 1; t /= 2)
+        if (nColBlocks * divru(tiles, t) >= 512)
+            return t;
+    return 1;
+}
 
 /* Double solvers: F[y][c] = sum_{k < K} q[y][k] B[k][c] with B row-major, as it
  * is stored (the dense annealer's J, the bipartite one's J or J^T).
@@ -381,9 +356,10 @@ __device__ __forceinline__ uint2 spinsFP8(uint32_t bits) {
  * k = 256 s + 64 g + 32 d + e, e < 32: spin word 8 s + 2 g + d of the row,
  * bit e -- so each lane's A operand for a whole super-block is the 8-byte
  * pair of words (8 s + 2 g, 8 s + 2 g + 1) of its row, loaded directly. */
+template <int T>
 __device__ __forceinline__ void refreshFP8Block(const uint4 *frag, const float *colScale, const uint32_t *Qbits,
-                                                int K, int m, int Nw, int ldF, float *F, int cb, RedTile *red,
-                                                const uint2 *lut) {
+                                                int K, int m, int Nw, int ldF, float *F, int cb, int y0,
+                                                RedTile<T> *red, const uint2 *lut) {
     const int lane = threadIdx.x % kWave;
     const int w = threadIdx.x / kWave;
     const int c = lane & 15, g = lane >> 4;
@@ -391,86 +367,64 @@ __device__ __forceinline__ void refreshFP8Block(const uint4 *frag, const float *
     const int nS = nK / kDepth8;
     const int sOff = (int)(((long long)cb * 3) % nS);
     const uint4 *fb = frag + (size_t)cb * nK * 2 * kWave + lane;
-    for (int y0 = 0; y0 < m; y0 += kRowsPerPass) {
-        f32x4 acc[kTiles];
+    f32x4 acc[T];
 #pragma unroll
-        for (int t = 0; t < kTiles; ++t)
-            acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        uint4 b0[2][kDepth8], b1[2][kDepth8];
-        uint2 qv[2][kTiles];
-        auto fetch = [&](int buf, int l) {
-            int s = l + sOff;
-            if (s >= nS)
-                s -= nS;
+    for (int t = 0; t < T; ++t)
+        acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    uint4 b0[2][kDepth8], b1[2][kDepth8];
+    uint2 qv[2][T];
+    auto fetch = [&](int buf, int l) {
+        int s = l + sOff;
+        if (s >= nS)
+            s -= nS;
 #pragma unroll
-            for (int d = 0; d < kDepth8; ++d) {
-                const uint4 *p = fb + (size_t)(s * kDepth8 + d) * 2 * kWave;
-                b0[buf][d] = p[0];
-                b1[buf][d] = p[kWave];
-            }
-#pragma unroll
-            for (int t = 0; t < kTiles; ++t) {
-                const int y = y0 + 16 * t + c;
-                const uint2 v = *reinterpret_cast<const uint2 *>(Qbits + (size_t)(y < m ? y : m - 1) * Nw + 8 * s + 2 * g);
-                qv[buf][t] = (y < m) ? v : uint2{0u, 0u};
-            }
-        };
-        /* A operands (four table reads per tile) are gathered one group of
-         * four tiles ahead of the MFMAs that use them */
-        constexpr int kGroups = kTiles / 4;
-        auto gather = [&](int buf, int step, i32x8 aop[4]) {
-            const int d = step / kGroups, t0 = (step % kGroups) * 4;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int t = t0 + u;
-                if (y0 + 16 * t < m) { /* wave-uniform */
-                    const uint32_t word = d == 0 ? qv[buf][t].x : qv[buf][t].y;
-                    const uint2 l0 = lut[word & 0xffu], l1 = lut[(word >> 8) & 0xffu];
-                    const uint2 l2 = lut[(word >> 16) & 0xffu], l3 = lut[word >> 24];
-                    aop[u] = i32x8{(int)l0.x, (int)l0.y, (int)l1.x, (int)l1.y,
-                                   (int)l2.x, (int)l2.y, (int)l3.x, (int)l3.y};
-                }
-            }
-        };
-        auto compute = [&](int buf) {
-            i32x8 aop[2][4];
-            gather(buf, 0, aop[0]);
-#pragma unroll
-            for (int step = 0; step < kDepth8 * kGroups; ++step) {
-                if (step + 1 < kDepth8 * kGroups)
-                    gather(buf, step + 1, aop[(step + 1) & 1]);
-                const int d = step / kGroups, t0 = (step % kGroups) * 4;
-                const uint4 x0 = b0[buf][d], x1 = b1[buf][d];
-                const i32x8 bop = {(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w,
-                                   (int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int t = t0 + u;
-                    if (y0 + 16 * t < m) /* wave-uniform */
-                        acc[t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(aop[step & 1][u], bop, acc[t], 0, 0,
-                                                                                  0, kE4M3Unit, 0, kE4M3Unit);
-                }
-            }
-        };
-        for (int l = w; l < nS; l += 2 * kSplitK) {
-            if (l == w)
-                fetch(0, l);
-            if (l + kSplitK < nS)
-                fetch(1, l + kSplitK);
-            compute(0);
-            if (l + kSplitK >= nS)
-                break;
-            if (l + 2 * kSplitK < nS)
-                fetch(0, l + 2 * kSplitK);
-            compute(1);
+        for (int d = 0; d < kDepth8; ++d) {
+            const uint4 *p = fb + (size_t)(s * kDepth8 + d) * 2 * kWave;
+            b0[buf][d] = p[0];
+            b1[buf][d] = p[kWave];
         }
 #pragma unroll
-        for (int t = 0; t < kTiles; ++t)
+        for (int t = 0; t < T; ++t) {
+            const int y = y0 + 16 * t + c;
+            qv[buf][t] = *reinterpret_cast<const uint2 *>(Qbits + (size_t)(y < m ? y : m - 1) * Nw + 8 * s + 2 * g);
+        }
+    };
+    auto compute = [&](int buf) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                red[w][4 * t + r][lane] = acc[t][r];
-        reduceStore(red, y0, m, cb, ldF, F, colScale);
+        for (int d = 0; d < kDepth8; ++d) {
+            const uint4 x0 = b0[buf][d], x1 = b1[buf][d];
+            const i32x8 bop = {(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w,
+                               (int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
+            /* A operands (four table reads per tile) */
+            i32x8 aop[T];
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                const uint32_t word = d == 0 ? qv[buf][t].x : qv[buf][t].y;
+                const uint2 l0 = lut[word & 0xffu], l1 = lut[(word >> 8) & 0xffu];
+                const uint2 l2 = lut[(word >> 16) & 0xffu], l3 = lut[word >> 24];
+                aop[t] = i32x8{(int)l0.x, (int)l0.y, (int)l1.x, (int)l1.y,
+                               (int)l2.x, (int)l2.y, (int)l3.x, (int)l3.y};
+            }
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+                if (y0 + 16 * t < m) /* wave-uniform */
+                    acc[t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(aop[t], bop, acc[t], 0, 0, 0, kE4M3Unit,
+                                                                              0, kE4M3Unit);
+        }
+    };
+    for (int l = w; l < nS; l += 2 * kSplitK) {
+        if (l == w)
+            fetch(0, l);
+        if (l + kSplitK < nS)
+            fetch(1, l + kSplitK);
+        compute(0);
+        if (l + kSplitK >= nS)
+            break;
+        if (l + 2 * kSplitK < nS)
+            fetch(0, l + 2 * kSplitK);
+        compute(1);
     }
+    reduceStore<T>(acc, red, y0, m, cb, ldF, F, colScale);
 }
 
 __device__ __forceinline__ void fillLutFP8(uint2 *lut) {
@@ -479,17 +433,21 @@ __device__ __forceinline__ void fillLutFP8(uint2 *lut) {
     __syncthreads();
 }
 
+template <int T>
 __global__ __launch_bounds__(kBlockThreads) void fieldRefreshFP8Kernel(const uint4 *frag, const float *colScale,
-                                                                       const uint32_t *Qbits, int K, int m, int Nw,
-                                                                       int ldF, float *F) {
-    __shared__ float red[kSplitK][kTiles * 4][kWave]; /* 64 KiB */
-    __shared__ uint2 lut[256];                        /* 2 KiB */
+                                                                       const uint32_t *Qbits, int nColBlocks,
+                                                                       int nGroups, int K, int m, int Nw, int ldF,
+                                                                       float *F) {
+    __shared__ RedTile<T> red[kSplitK];
+    __shared__ uint2 lut[256]; /* 2 KiB */
+    int cb, y0;
+    blockTile(blockIdx.x, nColBlocks, nGroups, 16 * T, cb, y0);
     fillLutFP8(lut);
-    refreshFP8Block(frag, colScale, Qbits, K, m, Nw, ldF, F, blockIdx.x, red, lut);
+    refreshFP8Block<T>(frag, colScale, Qbits, K, m, Nw, ldF, F, cb, y0, red, lut);
 }
 
-/* Many GEMMs of one form in one launch: block b runs column block
- * b - blockStart[j] of job j, blockStart[j] <= b < blockStart[j + 1]. */
+/* Many GEMMs of one form in one launch: block b runs block b - blockStart[j] of
+ * job j, blockStart[j] <= b < blockStart[j + 1]. */
 __device__ __forceinline__ int jobOfBlock(const int *blockStart, int nJobs) {
     int lo = 0, hi = nJobs - 1;
     const int b = blockIdx.x;
@@ -506,32 +464,22 @@ __device__ __forceinline__ int jobOfBlock(const int *blockStart, int nJobs) {
 template <int FORM>
 __global__ __launch_bounds__(kBlockThreads) void fieldRefreshGroupedKernel(const FieldGemmJob *jobs,
                                                                            const int *blockStart, int nJobs) {
-    __shared__ float red[kSplitK][kTiles * 4][kWave];
+    __shared__ RedTile<kGroupedTiles> red[kSplitK];
     __shared__ uint4 lut[256];
     const int j = jobOfBlock(blockStart, nJobs);
     const FieldGemmJob jb = jobs[j];
-    const int cb = (int)blockIdx.x - blockStart[j];
-    if constexpr (FORM == fieldBF16x2) {
-        fillLutBF16(lut);
-        /* the split as a template argument: each path allocates its own registers */
-        if (bf16ColSplit(jb.K))
-            refreshBF16Block<2, true>(reinterpret_cast<const uint4 *>(jb.frag), jb.Qbits, jb.K, jb.m, jb.Nw, jb.ldF,
-                                      jb.F, cb, red, lut);
-        else
-            refreshBF16Block<2, false>(reinterpret_cast<const uint4 *>(jb.frag), jb.Qbits, jb.K, jb.m, jb.Nw, jb.ldF,
-                                       jb.F, cb, red, lut);
-    } else if constexpr (FORM == fieldFP8) {
+    const uint4 *frag = reinterpret_cast<const uint4 *>(jb.frag);
+    int cb, y0;
+    blockTile((int)blockIdx.x - blockStart[j], jb.nCols / 16, divru(jb.m, 16 * kGroupedTiles), 16 * kGroupedTiles, cb,
+              y0);
+    if constexpr (FORM == fieldFP8) {
         fillLutFP8(reinterpret_cast<uint2 *>(lut));
-        refreshFP8Block(reinterpret_cast<const uint4 *>(jb.frag), jb.colScale, jb.Qbits, jb.K, jb.m, jb.Nw, jb.ldF,
-                        jb.F, cb, red, reinterpret_cast<const uint2 *>(lut));
+        refreshFP8Block<kGroupedTiles>(frag, jb.colScale, jb.Qbits, jb.K, jb.m, jb.Nw, jb.ldF, jb.F, cb, y0, red,
+                                       reinterpret_cast<const uint2 *>(lut));
     } else {
         fillLutBF16(lut);
-        if (bf16ColSplit(jb.K))
-            refreshBF16Block<3, true>(reinterpret_cast<const uint4 *>(jb.frag), jb.Qbits, jb.K, jb.m, jb.Nw, jb.ldF,
-                                      jb.F, cb, red, lut);
-        else
-            refreshBF16Block<3, false>(reinterpret_cast<const uint4 *>(jb.frag), jb.Qbits, jb.K, jb.m, jb.Nw, jb.ldF,
-                                       jb.F, cb, red, lut);
+        refreshBF16Block<FORM == fieldBF16x2 ? 2 : 3, kGroupedTiles>(frag, jb.Qbits, jb.K, jb.m, jb.Nw, jb.ldF, jb.F,
+                                                                     cb, y0, red, lut);
     }
 }
 
@@ -631,9 +579,7 @@ void fieldRefreshGrouped(int fieldFormat, const FieldGemmJob *d_jobs, const int 
     HIP_CHECK(hipGetLastError());
 }
 
-int fieldGemmJobBlocks(const FieldGemmJob &j, int fieldFormat) {
-    return j.nCols / (fieldFormat != fieldFP8 && bf16ColSplit(j.K) ? 16 * kSplitK : 16);
-}
+int fieldGemmJobBlocks(const FieldGemmJob &j) { return j.nCols / 16 * divru(j.m, 16 * kGroupedTiles); }
 
 void checkFieldGemmJob(const FieldGemmJob &j, int fieldFormat) {
     checkGemm(j.nCols, j.K, j.K, j.Nw);
@@ -647,8 +593,11 @@ void fieldRefreshFP8(const uint8_t *d_frag, size_t fragElems, const float *d_col
     SQ_THROW_IF(ldF < nCols, "field GEMM: output stride %d < %d columns", ldF, nCols);
     SQ_THROW_IF(fragElems < fieldFragElemsFP8(nCols, K), "fp8 fragment buffer too small");
     SQ_THROW_IF(!d_colScale, "fp8 field GEMM: no column scales");
-    fieldRefreshFP8Kernel<<<nCols / 16, kBlockThreads, 0, stream>>>(reinterpret_cast<const uint4 *>(d_frag),
-                                                                    d_colScale, d_Qbits, K, m, Nw, ldF, d_F);
+    const int nColBlocks = nCols / 16, t = rowTilesFor(nColBlocks, m);
+    const int nGroups = divru(divru(m, 16), t);
+    auto *kernel = t == 4 ? fieldRefreshFP8Kernel<4> : t == 2 ? fieldRefreshFP8Kernel<2> : fieldRefreshFP8Kernel<1>;
+    kernel<<<nColBlocks * nGroups, kBlockThreads, 0, stream>>>(reinterpret_cast<const uint4 *>(d_frag), d_colScale, d_Qbits,
+                                                               nColBlocks, nGroups, K, m, Nw, ldF, d_F);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -681,8 +630,11 @@ void fieldRefreshBF16x2(const uint16_t *d_frag, size_t fragElems, const uint32_t
     checkGemm(nCols, K, K, Nw);
     SQ_THROW_IF(ldF < nCols, "field GEMM: output stride %d < %d columns", ldF, nCols);
     SQ_THROW_IF(fragElems < fieldFragElemsBF16x2(nCols, K), "bf16x2 fragment buffer too small");
-    fieldRefreshBF16x2Kernel<<<nCols / 16, kBlockThreads, 0, stream>>>(reinterpret_cast<const uint4 *>(d_frag),
-                                                                       d_Qbits, K, m, Nw, ldF, d_F);
+    const int nColBlocks = nCols / 16, t = rowTilesFor(nColBlocks, m);
+    const int nGroups = divru(divru(m, 16), t);
+    auto *kernel = t == 4 ? fieldRefreshBF16Kernel<2, 4> : t == 2 ? fieldRefreshBF16Kernel<2, 2> : fieldRefreshBF16Kernel<2, 1>;
+    kernel<<<nColBlocks * nGroups, kBlockThreads, 0, stream>>>(reinterpret_cast<const uint4 *>(d_frag), d_Qbits,
+                                                               nColBlocks, nGroups, K, m, Nw, ldF, d_F);
     HIP_CHECK(hipGetLastError());
 }
 
@@ -691,8 +643,11 @@ void fieldRefreshF32MFMA(const uint16_t *d_frag, size_t fragElems, const uint32_
     checkGemm(nCols, K, K, Nw);
     SQ_THROW_IF(ldF < nCols, "field GEMM: output stride %d < %d columns", ldF, nCols);
     SQ_THROW_IF(fragElems < fieldFragElemsF32(nCols, K), "fp32 fragment buffer too small");
-    fieldRefreshBF16x3Kernel<<<nCols / 16, kBlockThreads, 0, stream>>>(reinterpret_cast<const uint4 *>(d_frag),
-                                                                       d_Qbits, K, m, Nw, ldF, d_F);
+    const int nColBlocks = nCols / 16, t = rowTilesFor(nColBlocks, m);
+    const int nGroups = divru(divru(m, 16), t);
+    auto *kernel = t == 4 ? fieldRefreshBF16Kernel<3, 4> : t == 2 ? fieldRefreshBF16Kernel<3, 2> : fieldRefreshBF16Kernel<3, 1>;
+    kernel<<<nColBlocks * nGroups, kBlockThreads, 0, stream>>>(reinterpret_cast<const uint4 *>(d_frag), d_Qbits,
+                                                               nColBlocks, nGroups, K, m, Nw, ldF, d_F);
     HIP_CHECK(hipGetLastError());
 }
 

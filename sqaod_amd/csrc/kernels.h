@@ -159,7 +159,7 @@ struct FieldGemmJob {
 void checkFieldGemmJob(const FieldGemmJob &job, int fieldFormat);
 /* workgroups of a job in a grouped launch (the bf16 forms give a short
  * k-range four column blocks per workgroup) */
-int fieldGemmJobBlocks(const FieldGemmJob &job, int fieldFormat);
+int fieldGemmJobBlocks(const FieldGemmJob &job);
 void fieldRefreshGrouped(int fieldFormat, const FieldGemmJob *d_jobs, const int *d_blockStart, int nJobs,
                          int totalBlocks, hipStream_t stream);
 void buildFragFP8(const uint8_t *d_B8, int rows, int ld8, int nCols, int K, uint8_t *d_frag, size_t fragElems,

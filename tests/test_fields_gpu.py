@@ -91,3 +91,13 @@ def test_field_gemm_fp64(oracle, rocm, N, m):
     F, J = an.get_fields(), oracle.dense_hamiltonian(W)[1]
     bound = 2.0 * N * 2.0 ** -53 * np.abs(J).sum(axis=1)  # the host product's own rounding as well
     assert np.all(np.abs(F - host_fields(oracle, W, np.stack(an.get_q()))) <= bound)
+
+
+@pytest.mark.parametrize("form", ["fp32", "bf16x2", "fp8"])
+@pytest.mark.parametrize("N,m", [(1100, 210), (2040, 250)])
+def test_field_gemm_row_groups(oracle, rocm, form, N, m):
+    """Two (N=1100) and four (N=2040) row tiles per block, several row groups per
+    column block, the last one ragged: exact on integer problems."""
+    W = dense_int_W(N, SEED_BASE + N)
+    an = annealer(rocm, W, m, field_precision=form)
+    assert np.array_equal(an.get_fields().astype(np.float64), host_fields(oracle, W, np.stack(an.get_q())))
