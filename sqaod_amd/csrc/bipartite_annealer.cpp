@@ -427,6 +427,8 @@ void BipartiteGraphAnnealer<real>::halfStep(int side, real G, real beta, const u
     a.twoDivM = real(2.) / real(m_);
     a.coef = std::log(std::tanh(G * beta / real(m_))) / beta;
     a.beta = beta;
+    if (bipartiteFlips<real>(a, dev_->stream()))
+        return;
     a.sliceStep = 2;
     /* even slices (all of them when m is even; without m-1 when m is odd) */
     const int nEvenFirst = (m_ % 2 == 0) ? m_ / 2 : (m_ - 1) / 2;

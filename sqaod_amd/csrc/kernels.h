@@ -189,6 +189,11 @@ struct BGFlipArgs {
     const uint32_t *words;
     uint32_t key0, key1, ctr0, ctr1;
 };
+/* All phases of a coloring half-step in one launch (slice0 and sliceStep
+ * unused); false, with nothing launched, for SA and where phase by phase is
+ * the faster or only way. */
+template <class real>
+bool bipartiteFlips(const BGFlipArgs<real> &a, hipStream_t stream);
 template <class real>
 void bipartiteFlipPhase(const BGFlipArgs<real> &a, int nSlices, hipStream_t stream);
 

@@ -90,6 +90,28 @@ def test_bit_exact_float64_coloring(oracle, rocm):
     assert np.array_equal(q0, r0) and np.array_equal(q1, r1)
 
 
+@pytest.mark.parametrize("N0,N1,m", [
+    (7, 9, 2),           # part of a byte, one byte and a bit; both neighbours the same slice
+    (8, 33, 3),
+    (65, 1, 129),        # more spins than a block has threads
+    (3, 2, 16384),       # the most slices of one launch for all phases
+    (3, 2, 16385),       # phase by phase, odd
+    (16384, 2, 64),      # the most spins of one launch
+    (16385, 2, 64),      # phase by phase on one side only
+])
+def test_flip_launches_bit_exact(oracle, rocm, N0, N1, m):
+    """Integer couplings: every field is exact, so every spin equals the
+    oracle's, at low and high acceptance."""
+    b0, b1, W = int_problem(N0, N1, SEED_BASE + 700 + N0 + m)
+    an, ref = make_pair(rocm, oracle, b0, b1, W, m, np.float32)
+    for G, beta in ((5.0, 0.02), (1.0, 0.5), (0.1, 50.0)):
+        an.anneal_one_step(G, beta)
+        ref.anneal_one_step(G, beta)
+        q0, q1 = pair_arrays(an.get_q())
+        r0, r1 = ref.get_q()
+        assert np.array_equal(q0, r0) and np.array_equal(q1, r1), (G, beta)
+
+
 def test_hamiltonian_and_energy_against_oracle(oracle, rocm):
     """test_bipartite_graph_annealer.py:64-86: get_hamiltonian equals the
     formulas, set_hamiltonian round-trips; energies equal the FP64 oracle."""
