@@ -312,6 +312,10 @@ int sqaod_rocm_formulas_assign_device(sqaod_rocm_formulas *f, sqaod_rocm_device 
 /* dense_graph_(batch_)calculate_E (:89-157): E[b] = x_b^T W x_b, x int8 nBatch x N */
 int sqaod_rocm_dense_graph_batch_calculate_E(sqaod_rocm_formulas *f, int dtype, void *E, const void *W, int N,
                                              const int8_t *x, int nBatch);
+/* The same with *symmetric = 1 where W equals its transpose; else *symmetric = 0
+ * and E is undefined (the check runs on the device beside the upload). */
+int sqaod_rocm_dense_graph_batch_calculate_E_if_symmetric(sqaod_rocm_formulas *f, int dtype, void *E, const void *W,
+                                                          int N, const int8_t *x, int nBatch, int *symmetric);
 /* dense_graph_calculate_hamiltonian (:159-201): h[N], J[N x N], c[1] */
 int sqaod_rocm_dense_graph_calculate_hamiltonian(sqaod_rocm_formulas *f, int dtype, void *h, void *J, void *c,
                                                  const void *W, int N);

@@ -27,6 +27,25 @@ def _check_bipartite(b0, b1, W):
 
 # dense graph
 
+# From this size on the device compares W with its transpose, beside the energies:
+# a call on 16 float32 states, host / device, is 69 / 85 us at N = 192, 108 / 91 at
+# 256, 380 / 158 at 512 (float64 88 / 92, 139 / 101, 598 / 226).
+_DEVICE_SYMMETRY_N = 256
+
+
+def _energies_if_symmetric(cext, cobj, W, x, dtype):
+    """E[b] = x_b^T W x_b in one device call, or None where the general path has
+    to look at the inputs: W small, not square or not equal to its transpose,
+    x of another length."""
+    if not isinstance(W, np.ndarray) or W.ndim != 2 or W.shape[0] != W.shape[1] or W.shape[0] < _DEVICE_SYMMETRY_N:
+        return None
+    x = _batch(x)
+    if x.ndim != 2 or x.shape[0] == 0 or x.shape[1] != W.shape[0]:
+        return None
+    E = np.empty((x.shape[0]), dtype)
+    return E if cext.dense_graph_batch_calculate_E_if_symmetric(cobj, E, W, x, dtype) else None
+
+
 def dense_graph_calculate_E(cext, cobj, W, x, dtype):
     W = common.symmetrize(common.fix_type(W, dtype))
     _check_qubo(W)
@@ -39,7 +58,11 @@ def dense_graph_calculate_E(cext, cobj, W, x, dtype):
 
 
 def dense_graph_batch_calculate_E(cext, cobj, W, x, dtype):
-    W = common.symmetrize(common.fix_type(W, dtype))
+    W = common.fix_type(W, dtype)
+    E = _energies_if_symmetric(cext, cobj, W, x, dtype)
+    if E is not None:
+        return E
+    W = common.symmetrize(W)
     _check_qubo(W)
     x = _batch(x)
     if x.shape[1] != W.shape[0]:

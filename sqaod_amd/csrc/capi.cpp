@@ -1166,6 +1166,17 @@ int sqaod_rocm_dense_graph_batch_calculate_E(sqaod_rocm_formulas *f, int dtype, 
     });
 }
 
+int sqaod_rocm_dense_graph_batch_calculate_E_if_symmetric(sqaod_rocm_formulas *f, int dtype, void *E, const void *W,
+                                                          int N, const int8_t *x, int nBatch, int *symmetric) {
+    return guarded([&] {
+        SQ_THROW_IF(!E || !W || !x || !symmetric, "null input");
+        withFormulas(f, dtype, [&](auto &s) {
+            using real = SQ_REAL(s);
+            *symmetric = s.denseCalculateEIfSymmetric(static_cast<real *>(E), static_cast<const real *>(W), N, x, nBatch);
+        });
+    });
+}
+
 int sqaod_rocm_dense_graph_calculate_hamiltonian(sqaod_rocm_formulas *f, int dtype, void *h, void *J, void *c,
                                                  const void *W, int N) {
     return guarded([&] {

@@ -35,7 +35,7 @@ Device &Formulas<real>::device() {
 template <class real>
 void Formulas<real>::run(QuadFormArgs<real> a, const real *A, size_t nA, const real *lin0, size_t n0,
                          const real *lin1, size_t n1, const int8_t *U, size_t nU, const int8_t *V, size_t nV,
-                         real *E, int nOut) {
+                         real *E, int nOut, bool *symmetric) {
     Device &dev = device();
     hipStream_t st = dev.stream();
     DevBuf<real> dA, d0, d1, dE;
@@ -65,11 +65,21 @@ void Formulas<real>::run(QuadFormArgs<real> a, const real *A, size_t nA, const r
         a.lin1 = d1.ptr;
     }
     a.E = dE.ptr;
+    DevBuf<int> dAsymmetric;
+    int asymmetric = 0;
+    if (symmetric) {
+        dAsymmetric.allocate(1);
+        symmetricCheck<real>(dA.ptr, a.nu, dAsymmetric.ptr, st);
+    }
     DevBuf<unsigned char> dWork;
     dWork.allocate(quadFormWorkBytes(a.nu, a.nv, a.nV, a.twoD != 0));
     quadForm<real>(a, nOut, dWork.ptr, dWork.n, st);
     HIP_CHECK(hipMemcpyAsync(E, dE.ptr, (size_t)nOut * sizeof(real), hipMemcpyDeviceToHost, st));
+    if (symmetric)
+        HIP_CHECK(hipMemcpyAsync(&asymmetric, dAsymmetric.ptr, sizeof(int), hipMemcpyDeviceToHost, st));
     dev.synchronize();
+    if (symmetric)
+        *symmetric = !asymmetric;
 }
 
 template <class real>
@@ -82,6 +92,19 @@ void Formulas<real>::denseCalculateE(real *E, const real *W, int N, const int8_t
     a.nu = a.nv = N;
     a.nV = nBatch;
     run(a, W, (size_t)N * N, nullptr, 0, nullptr, 0, x, (size_t)N * nBatch, x, 0, E, nBatch);
+}
+
+template <class real>
+bool Formulas<real>::denseCalculateEIfSymmetric(real *E, const real *W, int N, const int8_t *x, int nBatch) {
+    SQ_THROW_IF(N <= 0 || nBatch <= 0, "bad shape N=%d, batch=%d", N, nBatch);
+    QuadFormArgs<real> a{};
+    a.cst = 0.;
+    a.sgn = 1.;
+    a.nu = a.nv = N;
+    a.nV = nBatch;
+    bool symmetric = false;
+    run(a, W, (size_t)N * N, nullptr, 0, nullptr, 0, x, (size_t)N * nBatch, x, 0, E, nBatch, &symmetric);
+    return symmetric;
 }
 
 template <class real>

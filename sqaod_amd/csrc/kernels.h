@@ -444,6 +444,11 @@ size_t quadFormWorkBytes(int nu, int nv, int nV, bool twoD);
 template <class real>
 void quadForm(const QuadFormArgs<real> &a, int nOut, void *d_work, size_t workBytes, hipStream_t stream);
 
+/* *d_asymmetric = 1 if A (N x N) differs from its transpose anywhere, else 0
+ * (not for a stream being captured). */
+template <class real>
+void symmetricCheck(const real *d_A, int N, int *d_asymmetric, hipStream_t stream);
+
 /* sum_y q_y . q_(y+1)%m (the Trotter coupling of getSystemE), in double. */
 void spinDotSum(const uint32_t *d_Qbits, int N, int m, int Nw, double *d_out, hipStream_t stream);
 

@@ -586,6 +586,8 @@ public:
     void assignDevice(Device &dev);
     /* x, q: nBatch rows of N int8; E: nBatch */
     void denseCalculateE(real *E, const real *W, int N, const int8_t *x, int nBatch);
+    /* The same where W equals its transpose; else returns false, E undefined. */
+    bool denseCalculateEIfSymmetric(real *E, const real *W, int N, const int8_t *x, int nBatch);
     void denseHamiltonian(real *h, real *J, real *c, const real *W, int N);
     void denseCalculateEFromSpin(real *E, const real *h, const real *J, real c, const int8_t *q, int N, int nBatch);
     /* W, J: N1 x N0; x0: nBatch0 x N0, x1: nBatch1 x N1; E: nBatch0 (pairs)
@@ -600,7 +602,7 @@ public:
 private:
     Device &device();
     void run(QuadFormArgs<real> a, const real *A, size_t nA, const real *lin0, size_t n0, const real *lin1,
-             size_t n1, const int8_t *U, size_t nU, const int8_t *V, size_t nV, real *E, int nOut);
+             size_t n1, const int8_t *U, size_t nU, const int8_t *V, size_t nV, real *E, int nOut, bool *symmetric = nullptr);
     Device *dev_ = nullptr;
 };
 

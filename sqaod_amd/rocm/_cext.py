@@ -104,6 +104,8 @@ _SIGS = {
     "sqaod_rocm_formulas_delete": (_i32, [_vp]),
     "sqaod_rocm_formulas_assign_device": (_i32, [_vp, _vp]),
     "sqaod_rocm_dense_graph_batch_calculate_E": (_i32, [_vp, _i32, _vp, _vp, _i32, _vp, _i32]),
+    "sqaod_rocm_dense_graph_batch_calculate_E_if_symmetric": (_i32, [_vp, _i32, _vp, _vp, _i32, _vp, _i32,
+                                                                     ctypes.POINTER(_i32)]),
     "sqaod_rocm_dense_graph_calculate_hamiltonian": (_i32, [_vp, _i32, _vp, _vp, _vp, _vp, _i32]),
     "sqaod_rocm_dense_graph_batch_calculate_E_from_spin": (_i32, [_vp, _i32, _vp, _vp, _vp, _vp, _vp, _i32, _i32]),
     "sqaod_rocm_bipartite_graph_batch_calculate_E": (_i32, [_vp, _i32, _vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp,
@@ -755,6 +757,14 @@ class _Formulas:
     def dense_graph_batch_calculate_E(cobj, E, W, x, dtype):
         _check(_lib.sqaod_rocm_dense_graph_batch_calculate_E(cobj, _dt(dtype), _ptr(E), _ptr(W), W.shape[0], _ptr(x),
                                                              x.shape[0]))
+
+    @staticmethod
+    def dense_graph_batch_calculate_E_if_symmetric(cobj, E, W, x, dtype):
+        """The same where W equals its transpose; else False, E undefined."""
+        symmetric = _i32()
+        _check(_lib.sqaod_rocm_dense_graph_batch_calculate_E_if_symmetric(
+            cobj, _dt(dtype), _ptr(E), _ptr(W), W.shape[0], _ptr(x), x.shape[0], ctypes.byref(symmetric)))
+        return bool(symmetric.value)
 
     @staticmethod
     def dense_graph_calculate_E(cobj, E, W, x, dtype):

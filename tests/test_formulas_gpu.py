@@ -167,3 +167,33 @@ def test_bipartite_energy_tiles(F, dtype, N0, N1, B0, B1):
     E = F.bipartite_graph_batch_calculate_E_2d(b0, b1, W, x0, x1, dtype)
     on = x1[:, 2].astype(bool)
     assert np.all(np.isposinf(E[on])) and np.array_equal(E[~on], exact[~on].astype(dtype))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("N", [255, 256, 257, 288, 300])  # the host's check, then the device's by tiles of 32
+def test_dense_energy_of_unsymmetric_matrices(F, dtype, N):
+    """What counts as symmetric does not depend on where W is compared: one
+    element off by an ulp is taken from the upper triangle, one triangle is
+    halved, anything else (NaN too) is refused.  Integer values: sums exact."""
+    rng = np.random.default_rng(SEED_BASE + N)
+    upper = np.triu(rng.integers(-8, 9, (N, N))).astype(dtype)
+    W = upper + np.triu(upper, 1).T
+    x = rng.integers(0, 2, (3, N)).astype(np.int8)
+    xd = x.astype(np.float64)
+    E = np.einsum("bi,ij,bj->b", xd, W.astype(np.float64), xd)
+    assert np.array_equal(F.dense_graph_batch_calculate_E(W, x, dtype), E)
+    assert np.array_equal(F.dense_graph_batch_calculate_E(upper, x, dtype),
+                          np.einsum("bi,ij,bj->b", xd, upper.astype(np.float64), xd))
+    for i, j in [(1, 0), (N - 1, 0), (N - 1, N - 2), (33, 31), (0, N - 1), (N // 2, N // 2 - 1)]:
+        ulp = W.copy()
+        ulp[max(i, j), min(i, j)] = np.nextafter(W[i, j], dtype(100.))
+        assert np.array_equal(F.dense_graph_batch_calculate_E(ulp, x, dtype), E), (i, j)
+        for bad in (W[i, j] + 1, np.nan):
+            off = W.copy()
+            off[i, j] = bad
+            with pytest.raises(RuntimeError):
+                F.dense_graph_batch_calculate_E(off, x, dtype)
+    off = W.copy()
+    off[N - 1, N - 1] = np.nan
+    with pytest.raises(RuntimeError):
+        F.dense_graph_batch_calculate_E(off, x, dtype)
