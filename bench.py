@@ -474,7 +474,7 @@ def main():
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": traffic,
             "traffic_frac": (traffic / sweep_s / 1e9 / HBM_PEAK_GBS) if traffic else None,
-            "kernel": "denseSweepKernel",
+            "kernel": "denseSweepTeamKernel",
             "algorithmic_bytes_per_launch": algo_per_launch,
             "note": "achieved = the local-field sweep's algorithmic bytes per launch (stream, decisions, fields, "
                     "spins, one J row per accepted flip at the measured flip count) / the sweep's average "
