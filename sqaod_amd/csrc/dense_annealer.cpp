@@ -602,6 +602,7 @@ void DenseGraphAnnealer<real>::prepare() {
     d_P_.allocate((size_t)m_ * ldP_);
     HIP_CHECK(hipMemsetAsync(d_P_.ptr, 0, d_P_.bytes(), dev_->stream()));
     tag_ = 0;
+    teamTag_ = 0;
     d_E_.allocate((size_t)m_);
     ensureEnergyPlanes();
     d_spinDot_.allocate(1);
@@ -928,8 +929,13 @@ void DenseGraphAnnealer<real>::annealOneStep(real G, real beta) {
     if (profile_)
         phaseBegin(2, pe);
     if (teamS > 0 && a.multiBufs < 2) {
-        if (a.tag % kTeamTagPeriod == 0) /* its words' tags start over */
+        /* its words' tags count the team's sweeps alone: other kernels may run any
+         * number of sweeps in between without touching the words */
+        if (teamTag_ == kTeamTagPeriod) {
+            teamTag_ = 0;
             HIP_CHECK(hipMemsetAsync(d_P_.ptr, 0, d_P_.bytes(), dev_->stream()));
+        }
+        a.tag = ++teamTag_;
         denseSweepTeam<real>(a, teamS, dev_->maxLdsPerBlock(), direct, dev_->numCUs(), dev_->stream());
     } else {
         denseSweep<real>(a, plainSweep_, sweepFormat, S, direct, dev_->numCUs(), dev_->stream());

@@ -313,8 +313,8 @@ void launchSweep(void *kernel, int nBlocks, int threads, size_t lds, void **karg
 
 /* The local-field sweep (float: rows of args.J; double) by a team of four waves
  * per slice, each batch ending at its first flip (dense_sweep_team.hip).
- * args.P: m rows of args.ldP >= teamWordStride(N) words, cleared before the first
- * sweep and every kTeamTagPeriod sweeps (args.tag % kTeamTagPeriod == 0). */
+ * args.P: m rows of args.ldP >= teamWordStride(N) words; args.tag: 1 to
+ * kTeamTagPeriod, no tag twice without P cleared in between. */
 constexpr uint32_t kTeamTagPeriod = 2047;
 int teamWordStride(int N);
 /* Slices per block (asked: 0 to choose), 0 where the sweep does not fit. */

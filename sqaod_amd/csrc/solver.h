@@ -225,6 +225,7 @@ private:
     unsigned long long seed_ = 0;
     unsigned long long sweepIdx_ = 0;
     uint32_t tag_ = 0;
+    uint32_t teamTag_ = 0; /* of the last team sweep since the words of P were cleared */
     real c_ = 0;
 
     /* preferences beyond the reference's */

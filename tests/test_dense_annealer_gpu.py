@@ -463,6 +463,21 @@ def test_team_sweep_bit_exact(oracle, rocm, N, m, spb, dtype, algo):
     assert np.array_equal(an.get_E(), ora.calculate_E())
 
 
+def test_team_sweep_after_a_tag_period_of_others(oracle, rocm):
+    """A team sweep a whole tag period (2047 sweeps) after the last one, the
+    sweeps in between by the one-wave kernel: no word of the old sweep counts."""
+    N, m = 24, 4
+    W = dense_int_W(N, SEED_BASE + 4)
+    ora, an = make_pair(oracle, rocm, W, m, seed=6, multi_flip="off")
+    for k in range(2060):
+        an.set_preferences(helper_wave="off" if 2 <= k < 2048 else "on")
+        G = 3.0 if k % 50 else 0.5
+        ora.anneal_one_step(G, 1.0)
+        an.anneal_one_step(G, 1.0)
+        if k >= 2040:
+            assert np.array_equal(q_of(an), ora.get_q()), k
+
+
 def test_team_sweep_past_its_tag_period(oracle, rocm):
     """More sweeps than the published words have tags (2047)."""
     N, m = 24, 4
