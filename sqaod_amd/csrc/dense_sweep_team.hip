@@ -674,7 +674,11 @@ __global__ __launch_bounds__(kTeamWaves *kTeamMaxSlices *kWave) void denseSweepT
         if (a.sa)
             return;
         const Neighbours nb = neighboursOf(y, a.m);
-        auto ownAt = [&](int n) { return n / S == b ? (int)(regions - lds) + r.bytes * (n - b * S) + r.own : -1; };
+        /* one slice a block keeps no words of its own: with m = 1, where it is its
+         * own neighbour, it reads them from memory as it would another block's */
+        auto ownAt = [&](int n) {
+            return S > 1 && n / S == b ? (int)(regions - lds) + r.bytes * (n - b * S) + r.own : -1;
+        };
         watcherLoop<real>(a, y, lds, region, r, ownAt(nb.n[0]), ownAt(nb.n[1]));
     } else {
         sweeperLoop<real>(a, y, expTab, hS, region, r);

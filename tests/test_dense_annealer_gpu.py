@@ -463,6 +463,24 @@ def test_team_sweep_bit_exact(oracle, rocm, N, m, spb, dtype, algo):
     assert np.array_equal(an.get_E(), ora.calculate_E())
 
 
+@pytest.mark.parametrize("N,spb,dtype", [(20, 0, np.float32), (100, 0, np.float32), (100, 0, np.float64),
+                                         (100, 2, np.float32), (300, 1, np.float32), (1100, 0, np.float32)])
+def test_one_slice_coloring_bit_exact(oracle, rocm, N, spb, dtype):
+    """prepare() selects SA for one slice; the coloring algorithm asked for
+    after it runs with the slice as its own neighbour on both sides.  Alone in
+    its block it keeps no decision words in LDS (spb 0 and 1), with room for
+    another slice it does (2)."""
+    W = dense_int_W(N, SEED_BASE + 13 * N)
+    ora, an = make_pair(oracle, rocm, W, 1, seed=17 + N, dtype=dtype, slices_per_block=spb)
+    ora.set_algorithm(3)
+    an.set_preferences(algorithm="coloring")
+    assert an.get_preferences()["algorithm"] == "coloring"
+    for G in schedule()[:160:5]:
+        ora.anneal_one_step(G, BETA)
+        an.anneal_one_step(G, BETA)
+        assert np.array_equal(q_of(an), ora.get_q())
+
+
 def test_team_sweep_after_a_tag_period_of_others(oracle, rocm):
     """A team sweep a whole tag period (2047 sweeps) after the last one, the
     sweeps in between by the one-wave kernel: no word of the old sweep counts."""
