@@ -591,7 +591,8 @@ void DenseGraphAnnealer<real>::prepare() {
         logf("Selecting %s as the default SA algorithm.", algorithmToString(algo_));
     }
     const size_t mN = (size_t)m_ * N_;
-    d_Q_.allocate((size_t)m_ * Nw_);
+    d_Q_.allocate(2 * (size_t)m_ * Nw_);
+    qBuf_ = 0;
     d_F_.allocate((size_t)m_ * Np_);
     d_X_.allocate(mN);
     d_U_.allocate(mN);
@@ -641,9 +642,9 @@ void DenseGraphAnnealer<real>::randomizeSpin() {
     ensureDevice();
     if (rngMT_) {
         mtGenerate(d_mt_.ptr, d_words_.ptr, (size_t)m_ * N_, dev_->stream());
-        spinsFromWords(d_words_.ptr, N_, N_, m_, Nw_, d_Q_.ptr, dev_->stream());
+        spinsFromWords(d_words_.ptr, N_, N_, m_, Nw_, spinWords(), dev_->stream());
     } else {
-        spinsFromPhilox(seed_, sweepIdx_++, N_, m_, Nw_, d_Q_.ptr, dev_->stream());
+        spinsFromPhilox(seed_, sweepIdx_++, N_, m_, Nw_, spinWords(), dev_->stream());
     }
     fieldsDirty_ = true;
     sweepsSinceSpinsSet_ = 0;
@@ -661,7 +662,7 @@ void DenseGraphAnnealer<real>::set_q(const int8_t *q, int N) {
         memcpy(&all[(size_t)y * N_], q, (size_t)N_);
     d_q8_.allocate(all.size());
     HIP_CHECK(hipMemcpyAsync(d_q8_.ptr, all.data(), all.size(), hipMemcpyHostToDevice, dev_->stream()));
-    packSpins(d_q8_.ptr, N_, m_, Nw_, d_Q_.ptr, dev_->stream());
+    packSpins(d_q8_.ptr, N_, m_, Nw_, spinWords(), dev_->stream());
     dev_->synchronize();
     fieldsDirty_ = true;
     sweepsSinceSpinsSet_ = 0;
@@ -678,7 +679,7 @@ void DenseGraphAnnealer<real>::set_qset(const int8_t *q, int m, int N) {
     prepare();
     d_q8_.allocate((size_t)m_ * N_);
     HIP_CHECK(hipMemcpyAsync(d_q8_.ptr, q, (size_t)m_ * N_, hipMemcpyHostToDevice, dev_->stream()));
-    packSpins(d_q8_.ptr, N_, m_, Nw_, d_Q_.ptr, dev_->stream());
+    packSpins(d_q8_.ptr, N_, m_, Nw_, spinWords(), dev_->stream());
     dev_->synchronize();
     fieldsDirty_ = true;
     sweepsSinceSpinsSet_ = 0;
@@ -721,26 +722,26 @@ void DenseGraphAnnealer<real>::refreshFields(bool always) {
     if (fieldFormat_ == fieldFP8) {
         /* the vector cross-check runs on J' as floats */
         if (mfma)
-            fieldRefreshFP8(d_frag8_.ptr, d_frag8_.n, d_scale_.ptr, d_Q_.ptr, Np_, Np_, m_, Nw_, Np_,
+            fieldRefreshFP8(d_frag8_.ptr, d_frag8_.n, d_scale_.ptr, spinWords(), Np_, Np_, m_, Nw_, Np_,
                             (float *)d_F_.ptr, dev_->stream());
         else
-            fieldRefresh<float>(d_Jsplit_.ptr, N_, Np_, Np_, d_Q_.ptr, m_, Nw_, Np_, (float *)d_F_.ptr, dev_->stream());
+            fieldRefresh<float>(d_Jsplit_.ptr, N_, Np_, Np_, spinWords(), m_, Nw_, Np_, (float *)d_F_.ptr, dev_->stream());
     } else if (fieldFormat_ == fieldBF16x2) {
         /* the vector cross-check runs on Jsplit = float(hi) + float(lo), the
          * same numbers as the two planes */
         if (mfma)
-            fieldRefreshBF16x2(d_frag16_.ptr, d_frag16_.n, d_Q_.ptr, Np_, Np_, m_, Nw_, Np_, (float *)d_F_.ptr,
+            fieldRefreshBF16x2(d_frag16_.ptr, d_frag16_.n, spinWords(), Np_, Np_, m_, Nw_, Np_, (float *)d_F_.ptr,
                                dev_->stream());
         else
-            fieldRefresh<float>(d_Jsplit_.ptr, N_, Np_, Np_, d_Q_.ptr, m_, Nw_, Np_, (float *)d_F_.ptr, dev_->stream());
+            fieldRefresh<float>(d_Jsplit_.ptr, N_, Np_, Np_, spinWords(), m_, Nw_, Np_, (float *)d_F_.ptr, dev_->stream());
     } else if (mfma && sizeof(real) == 8) {
-        fieldRefreshF64MFMA((const double *)d_J_.ptr, N_, Np_, Np_, d_Q_.ptr, m_, Nw_, Np_, (double *)d_F_.ptr,
+        fieldRefreshF64MFMA((const double *)d_J_.ptr, N_, Np_, Np_, spinWords(), m_, Nw_, Np_, (double *)d_F_.ptr,
                             dev_->stream());
     } else if (mfma) {
-        fieldRefreshF32MFMA(d_frag32_.ptr, d_frag32_.n, d_Q_.ptr, Np_, Np_, m_, Nw_, Np_, (float *)d_F_.ptr,
+        fieldRefreshF32MFMA(d_frag32_.ptr, d_frag32_.n, spinWords(), Np_, Np_, m_, Nw_, Np_, (float *)d_F_.ptr,
                             dev_->stream());
     } else {
-        fieldRefresh<real>(d_J_.ptr, N_, Np_, Np_, d_Q_.ptr, m_, Nw_, Np_, d_F_.ptr, dev_->stream());
+        fieldRefresh<real>(d_J_.ptr, N_, Np_, Np_, spinWords(), m_, Nw_, Np_, d_F_.ptr, dev_->stream());
     }
     fieldsDirty_ = false;
     stepsSinceRefresh_ = 0;
@@ -796,7 +797,8 @@ SweepArgs<real> DenseGraphAnnealer<real>::makeSweepArgs(real G, real beta) {
     a.ld8 = ld8_;
     a.h = d_h_.ptr;
     a.F = d_F_.ptr;
-    a.Qbits = d_Q_.ptr;
+    a.Qbits = spinWords();
+    a.Qout = d_Q_.ptr + (size_t)(1 - qBuf_) * m_ * Nw_;
     a.X = d_X_.ptr;
     a.U = d_U_.ptr;
     a.D = d_D_.ptr;
@@ -834,7 +836,7 @@ void DenseGraphAnnealer<real>::annealOneStepNaive(real G, real beta) {
     a.J = (fieldFormat_ != fieldF32) ? reinterpret_cast<const real *>(d_Jsplit_.ptr) : d_J_.ptr;
     a.h = d_h_.ptr;
     a.F = d_F_.ptr;
-    a.Qbits = d_Q_.ptr;
+    a.Qbits = spinWords();
     a.counters = d_counters_.ptr;
     if (rngMT_) {
         const int words = sizeof(real) == 4 ? 3 : 4;
@@ -855,6 +857,7 @@ void DenseGraphAnnealer<real>::annealOneStepNaive(real G, real beta) {
 
 template <class real>
 void DenseGraphAnnealer<real>::stepDone() {
+    qBuf_ = 1 - qBuf_;
     abortPending_ = true; /* the sweep reports an abort in h_abort_ itself */
     ++stepsSinceRefresh_;
     clearState(solSolutionAvailable);
@@ -995,7 +998,7 @@ FieldGemmJob DenseGraphAnnealer<real>::takeFieldGemmJob() {
              : fieldFormat_ == fieldFP8  ? (const void *)d_frag8_.ptr
                                          : (const void *)d_frag32_.ptr;
     j.colScale = d_scale_.ptr;
-    j.Qbits = d_Q_.ptr;
+    j.Qbits = spinWords();
     j.F = (float *)d_F_.ptr;
     j.nCols = Np_;
     j.K = Np_;
@@ -1047,10 +1050,10 @@ void DenseGraphAnnealer<real>::computeEnergies() {
      * takes the FP64 vector kernel */
     ensureEnergyPlanes();
     if (planes_.finite)
-        energyPlanes<real>(planes_, d_planes_.ptr, d_h_.ptr, nullptr, (double)c_, d_Q_.ptr, Nw_, d_Q_.ptr, Nw_, m_,
+        energyPlanes<real>(planes_, d_planes_.ptr, d_h_.ptr, nullptr, (double)c_, spinWords(), Nw_, spinWords(), Nw_, m_,
                            d_partial_.ptr, d_E_.ptr, dev_->stream());
     else
-        energyFP64<real>(d_J_.ptr, d_h_.ptr, (double)c_, d_Q_.ptr, N_, Np_, m_, Nw_, d_partial_.ptr, d_E_.ptr,
+        energyFP64<real>(d_J_.ptr, d_h_.ptr, (double)c_, spinWords(), N_, Np_, m_, Nw_, d_partial_.ptr, d_E_.ptr,
                          dev_->stream());
 }
 
@@ -1104,18 +1107,18 @@ double DenseGraphAnnealer<real>::formEnergyError() {
                 dev_->synchronize(); /* d_partial_ is reallocated */
                 d_partial_.allocate(energyPlanePartialCount(Lf, m_));
             }
-            energyPlanes<float>(Lf, frag.ptr, d_h_.ptr, nullptr, (double)c_, d_Q_.ptr, Nw_, d_Q_.ptr, Nw_, m_,
+            energyPlanes<float>(Lf, frag.ptr, d_h_.ptr, nullptr, (double)c_, spinWords(), Nw_, spinWords(), Nw_, m_,
                                 d_partial_.ptr, d_E_.ptr, dev_->stream());
             HIP_CHECK(hipMemcpyAsync(ef.data(), d_E_.ptr, (size_t)m_ * sizeof(double), hipMemcpyDeviceToHost,
                                      dev_->stream()));
             dev_->synchronize(); /* before frag is freed */
         } else {
-            energyFP64<real>(d_J_.ptr, d_h_.ptr, (double)c_, d_Q_.ptr, N_, Np_, m_, Nw_, d_partial_.ptr, d_E_.ptr,
+            energyFP64<real>(d_J_.ptr, d_h_.ptr, (double)c_, spinWords(), N_, Np_, m_, Nw_, d_partial_.ptr, d_E_.ptr,
                              dev_->stream());
             HIP_CHECK(hipMemcpyAsync(e.data(), d_E_.ptr, (size_t)m_ * sizeof(double), hipMemcpyDeviceToHost,
                                      dev_->stream()));
             dev_->synchronize();
-            energyFP64<real>(d_Jsplit_.ptr, d_h_.ptr, (double)c_, d_Q_.ptr, N_, Np_, m_, Nw_, d_partial_.ptr,
+            energyFP64<real>(d_Jsplit_.ptr, d_h_.ptr, (double)c_, spinWords(), N_, Np_, m_, Nw_, d_partial_.ptr,
                              d_E_.ptr, dev_->stream());
             HIP_CHECK(hipMemcpyAsync(ef.data(), d_E_.ptr, (size_t)m_ * sizeof(double), hipMemcpyDeviceToHost,
                                      dev_->stream()));
@@ -1135,7 +1138,7 @@ void DenseGraphAnnealer<real>::makeSolution() {
     throwErrorIfQNotSet();
     ensureDevice();
     d_q8_.allocate((size_t)m_ * N_);
-    unpackSpins(d_Q_.ptr, N_, m_, Nw_, d_q8_.ptr, dev_->stream());
+    unpackSpins(spinWords(), N_, m_, Nw_, d_q8_.ptr, dev_->stream());
     q_.resize((size_t)m_ * N_);
     HIP_CHECK(hipMemcpyAsync(q_.data(), d_q8_.ptr, q_.size(), hipMemcpyDeviceToHost, dev_->stream()));
     dev_->synchronize();
@@ -1177,7 +1180,7 @@ real DenseGraphAnnealer<real>::getSystemE(real G, real beta) {
     E = E / real(m_);
     if (isSQAAlgorithm(algo_)) {
         double dot = 0.;
-        spinDotSum(d_Q_.ptr, N_, m_, Nw_, d_spinDot_.ptr, dev_->stream());
+        spinDotSum(spinWords(), N_, m_, Nw_, d_spinDot_.ptr, dev_->stream());
         HIP_CHECK(hipMemcpyAsync(&dot, d_spinDot_.ptr, sizeof(double), hipMemcpyDeviceToHost, dev_->stream()));
         dev_->synchronize();
         real spinDotSum_ = (real)dot;
@@ -1214,7 +1217,7 @@ void DenseGraphAnnealer<real>::traceSystemE(real G, real beta) {
     const int sqa = isSQAAlgorithm(algo_) ? 1 : 0;
     real coef = real(0.);
     if (sqa) {
-        spinDotSum(d_Q_.ptr, N_, m_, Nw_, d_spinDot_.ptr, dev_->stream());
+        spinDotSum(spinWords(), N_, m_, Nw_, d_spinDot_.ptr, dev_->stream());
         coef = real(0.5) / beta * std::log(std::tanh(G * beta / real(m_)));
     }
     const real sgn = (om_ == optMaximize) ? real(-1.) : real(1.);

@@ -17,6 +17,7 @@
  */
 #include <algorithm>
 #include <cstring>
+#include <functional>
 #include <numeric>
 
 #include "solver.h"
@@ -188,7 +189,20 @@ void GroupedDenseStepper::run(Device &dev, const std::vector<DenseGraphAnnealer<
                 capacity * wpb, maxM);
     const int nBlocks = std::min(capacity, (nItems + wpb - 1) / wpb);
 
-    /* plan every step on the host, in the order annealOneStep takes them */
+    /* plan every step on the host, in the order annealOneStep takes them; what
+     * fails before the first launch leaves the instances where they were */
+    std::vector<std::pair<int, DenseGraphAnnealer<float>::StepState>> before;
+    for (int i : order)
+        before.emplace_back(i, inst[i]->stepState());
+    bool launched = false;
+    struct Restore {
+        std::function<void()> f;
+        ~Restore() { f(); }
+    } restore{[&] {
+        if (!launched)
+            for (auto &b : before)
+                inst[b.first]->setStepState(b.second);
+    }};
     struct StepLayout {
         size_t gj, gs, sj, ss, sa;
         int nGemm, gemmBlocks, streamBlocks;
@@ -303,10 +317,12 @@ void GroupedDenseStepper::run(Device &dev, const std::vector<DenseGraphAnnealer<
             HIP_CHECK(hipStreamEndCapture(st, &g));
             HIP_CHECK(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0));
             HIP_CHECK(hipEventRecord(e0, st));
+            launched = true;
             HIP_CHECK(hipGraphLaunch(ge, st));
             HIP_CHECK(hipEventRecord(e1, st));
         } else {
             HIP_CHECK(hipEventRecord(e0, st));
+            launched = true;
             launchAll();
             HIP_CHECK(hipEventRecord(e1, st));
         }
@@ -365,11 +381,11 @@ void DenseBatch::autotune(double G, double beta, int trialSteps) {
     auto restore = [&]() {
         for (size_t i = 0; i < inst_.size(); ++i) {
             auto *a = inst_[i];
+            a->setStepState(ss[i]); /* and with it which of its buffers holds the spins */
             const size_t nq = (size_t)a->numTrotters() * (a->paddedN() / 32),
                          nf = (size_t)a->numTrotters() * a->paddedN();
             HIP_CHECK(hipMemcpyAsync(a->spinWords(), snapQ.ptr + qOff[i], nq * 4, hipMemcpyDeviceToDevice, st));
             HIP_CHECK(hipMemcpyAsync(a->fields(), snapF.ptr + fOff[i], nf * 4, hipMemcpyDeviceToDevice, st));
-            a->setStepState(ss[i]);
         }
         HIP_CHECK(hipStreamSynchronize(st));
     };

@@ -996,7 +996,10 @@ __device__ __forceinline__ void sweepSlice(const SweepArgs<real> &a, const int y
         }
         for (int b = 0; b < Nw; b += kWave)
             if (b + lane < Nw)
-                a.Qbits[(long long)y * Nw + b + lane] = Qb[b + lane];
+                a.Qout[(long long)y * Nw + b + lane] = Qb[b + lane];
+    } else { /* the slice keeps its spins */
+        for (int b = lane; b < Nw; b += kWave)
+            a.Qout[(long long)y * Nw + b] = a.Qbits[(long long)y * Nw + b];
     }
     if (lane == 0 && a.counters) {
         atomicAdd(&a.counters[0], (unsigned long long)nFlips);
@@ -1238,6 +1241,7 @@ template <class real>
 void denseSweep(const SweepArgs<real> &args, bool plain, int fieldFormat, int slicesPerBlock, bool allowDirect,
                 int numCUs, hipStream_t stream) {
     SQ_THROW_IF(args.Np % 256 != 0, "padded N must be a multiple of 256");
+    SQ_THROW_IF(!args.Qout || args.Qout == args.Qbits, "the sweep needs a second spin buffer");
     SQ_THROW_IF(slicesPerBlock < 1 || slicesPerBlock > kMaxSlicesPerBlock, "slices per block out of range (1..%d)",
                 kMaxSlicesPerBlock);
     const bool fp8 = !plain && fieldFormat == fieldFP8;

@@ -352,6 +352,13 @@ __device__ __forceinline__ T inVector(T v) {
     return v;
 }
 
+/* A pointer to device memory that was itself loaded, for which the compiler would
+ * not know. */
+template <class T>
+__device__ __forceinline__ T *inGlobal(T *p) {
+    return (T *)(__attribute__((address_space(1))) T *)p;
+}
+
 /* The sweeper of slice y. */
 template <class real>
 __device__ __forceinline__ void sweeperLoop(const SweepArgs<real> &a, const int y, const uint64_t *expTab, const real *hS,
@@ -589,21 +596,33 @@ __device__ __forceinline__ void sweeperLoop(const SweepArgs<real> &a, const int 
     while (ctlLoad(ctl + kCtlDone) != rows)
         ;
     ctlStore(ctl + kCtlRows, kEnd);
+    /* the arguments, read anew: kept from the start, they would take scalar
+     * registers from the loop (double then spills some: 33.2 us a sweep against
+     * 32.7 at N=500, m=125) */
+    const auto *e = (const __attribute__((address_space(4))) SweepArgs<real> *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(e));
+    uint32_t *const Qout = inGlobal(e->Qout) + (long long)y * Nw;
     if (!aborted) {
+        real *const Fout = inGlobal(e->F) + (long long)y * Np;
 #pragma unroll 4
         for (int b = 0; b < Np; b += kWave * 4) {
             real v[4];
             ldsLoad4(F + b + lane * 4, v);
-            ldsStore4(a.F + (long long)y * Np + b + lane * 4, v); /* a plain vector store, here to global */
+            ldsStore4(Fout + b + lane * 4, v); /* a plain vector store, here to global */
         }
         for (int b = 0; b < Nw; b += kWave)
             if (b + lane < Nw)
-                a.Qbits[(long long)y * Nw + b + lane] = Qb[b + lane];
+                Qout[b + lane] = Qb[b + lane];
+    } else { /* the slice keeps its spins */
+        const uint32_t *const Qin = inGlobal(e->Qbits) + (long long)y * Nw;
+        for (int b = lane; b < Nw; b += kWave)
+            Qout[b] = Qin[b];
     }
-    if (lane == 0 && a.counters) {
-        atomicAdd(&a.counters[0], (unsigned long long)nFlips);
-        atomicAdd(&a.counters[1], (unsigned long long)nBatches);
-        atomicAdd(&a.counters[2], (unsigned long long)nBlocked);
+    unsigned long long *const counters = inGlobal(e->counters);
+    if (lane == 0 && counters) {
+        atomicAdd(&counters[0], (unsigned long long)nFlips);
+        atomicAdd(&counters[1], (unsigned long long)nBatches);
+        atomicAdd(&counters[2], (unsigned long long)nBlocked);
     }
 }
 
@@ -727,6 +746,7 @@ void denseSweepTeam(const SweepArgs<real> &args, int slicesPerBlock, size_t maxL
                 "team sweep: bad row of %d sites in %d", args.N, args.Np);
     SQ_THROW_IF(slicesPerBlock < 1 || slicesPerBlock > kTeamMaxSlices, "slices per block out of range (1..%d)",
                 kTeamMaxSlices);
+    SQ_THROW_IF(!args.Qout || args.Qout == args.Qbits, "the sweep needs a second spin buffer");
     SQ_THROW_IF(!args.P || args.ldP < teamWordStride(args.N), "team sweep: no decision words");
     const int nBlocks = divru(args.m, slicesPerBlock);
     int xcdRemap = (nBlocks % 8 == 0 && nBlocks >= 16) ? 1 : 0;

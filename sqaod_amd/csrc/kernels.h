@@ -272,7 +272,12 @@ struct SweepArgs {
     int ld8;
     const real *h;          /* Np */
     real *F;                /* m x Np, in/out */
-    uint32_t *Qbits;        /* m x Nw, in/out */
+    /* m x Nw: the spins before and after the sweep.  Two buffers, since nothing
+     * orders a slice's end before the start of its neighbours: those read its
+     * spins as they start, which may be after it has ended, and add the flips
+     * that it has published. */
+    const uint32_t *Qbits;
+    uint32_t *Qout;
     const uint32_t *X;      /* m x N sites */
     const real *U;          /* m x N uniforms */
     uint32_t *D;            /* m x N decisions (tag << 1 | flipped) */

@@ -196,7 +196,7 @@ size_t Server::estimateDenseBytes(int N, int m, int fieldFormat) {
         b += n * Np * 4 + n * ((Np + 1023) / 1024 * 1024) + Np * Np + Np * 8; /* J', rows, fragments, scales */
     else
         b += Np * Np * 4;                                           /* fp32 fragments */
-    b += (size_t)m * Np * 4 + 3 * (size_t)m * n * 4 + (size_t)m * Np / 8; /* F, X, U, D, Q */
+    b += (size_t)m * Np * 4 + 3 * (size_t)m * n * 4 + (size_t)m * Np / 4; /* F, X, U, D, Q (two buffers) */
     b += (size_t)m * (Np / 256 + 2) * 8 + (size_t)m * n;            /* energies, q for makeSolution */
     b += 6 * Np * Np + (size_t)m * (2048 + Np / 16) * 8;            /* energy planes (at most 6), partials */
     return b + b / 16 + ((size_t)1 << 20);

@@ -184,25 +184,27 @@ public:
     FieldGemmJob takeFieldGemmJob();         /* the step's field refresh, enqueued by the caller */
     AttemptStreamJob takeAttemptStreamJob(); /* the step's Philox streams (advances the sweep index) */
     SweepArgs<real> makeSweepArgs(real G, real beta);
-    void stepDone();
+    void stepDone(); /* the sweep is enqueued: its spins are the present ones */
     void checkStepAbort() { checkAbort(false); }
     int fieldFormat() const { return fieldFormat_; }
     int paddedN() const { return Np_; }
     int fp8RowStrideBytes() const { return ld8_; }
     Device *device() const { return dev_; }
     /* spins and fields, for snapshots around trial steps */
-    uint32_t *spinWords() { return d_Q_.ptr; }
+    uint32_t *spinWords() { return d_Q_.ptr + (size_t)qBuf_ * m_ * Nw_; }
     real *fields() { return d_F_.ptr; }
     struct StepState {
         unsigned long long sweepIdx;
         int stepsSinceRefresh;
         bool fieldsDirty;
+        int spinBuffer; /* which spinWords() is */
     };
-    StepState stepState() const { return {sweepIdx_, stepsSinceRefresh_, fieldsDirty_}; }
+    StepState stepState() const { return {sweepIdx_, stepsSinceRefresh_, fieldsDirty_, qBuf_}; }
     void setStepState(const StepState &s) {
         sweepIdx_ = s.sweepIdx;
         stepsSinceRefresh_ = s.stepsSinceRefresh;
         fieldsDirty_ = s.fieldsDirty;
+        qBuf_ = s.spinBuffer;
     }
 
 private:
@@ -282,7 +284,8 @@ private:
     DevBuf<float> d_scale_;     /* fp8 form: 2^a_i per row (Np, 1 past N) */
     DevBuf<int> d_rowExp_;
     int ld8_ = 0;
-    DevBuf<uint32_t> d_Q_, d_X_, d_D_, d_words_;
+    DevBuf<uint32_t> d_Q_, d_X_, d_D_, d_words_; /* d_Q_: two buffers of m x Nw spins */
+    int qBuf_ = 0; /* the present spins' */
     DevBuf<uint32_t> d_P_; /* the team sweep's published words, m x ldP_ */
     int ldP_ = 0;
     DevBuf<MTState> d_mt_;

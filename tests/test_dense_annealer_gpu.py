@@ -463,6 +463,50 @@ def test_team_sweep_bit_exact(oracle, rocm, N, m, spb, dtype, algo):
     assert np.array_equal(an.get_E(), ora.calculate_E())
 
 
+@pytest.mark.parametrize("prefs", [dict(), dict(helper_wave="off"), dict(helper_wave="off", multi_flip="2"),
+                                   dict(sweep="plain")], ids=["team", "one_wave", "multi_flip", "plain"])
+@pytest.mark.parametrize("N,m", [(5, 64), (16, 48), (32, 33), (61, 48)])
+def test_short_slices_over_many_blocks_bit_exact(oracle, rocm, N, m, prefs):
+    """A slice this short may end before a neighbour in another block has
+    started, which then reads its spins: those from before the sweep, to which
+    it adds the published flips."""
+    W = dense_int_W(N, SEED_BASE + 19 * N)
+    ora, an = make_pair(oracle, rocm, W, m, seed=23 + N, slices_per_block=1, **prefs)
+    for k, G in enumerate(schedule()):
+        ora.anneal_one_step(G, BETA)
+        an.anneal_one_step(G, BETA)
+        if k % 20 == 0:
+            assert np.array_equal(q_of(an), ora.get_q()), f"step {k}"
+    assert np.array_equal(q_of(an), ora.get_q())
+
+
+def test_spins_follow_through_changing_steps(oracle, rocm):
+    """A sweep leaves its spins in another buffer than it read, the naive step,
+    set_q and randomize_spin work on the present one: a mixed sequence of odd
+    lengths stays the serial CPU annealer's."""
+    N, m = 70, 6
+    W = dense_int_W(N, SEED_BASE + 29)
+    ora, an = make_pair(oracle, rocm, W, m, seed=37)
+    rng = np.random.default_rng(SEED_BASE)
+    for rep, steps in enumerate([1, 2, 3, 1, 4, 5]):
+        for name, code in (("coloring", 3), ("naive", 2)):
+            ora.set_algorithm(code)
+            an.set_preferences(algorithm=name)
+            for G in schedule()[rep * 20:rep * 20 + steps]:
+                ora.anneal_one_step(G, BETA)
+                an.anneal_one_step(G, BETA)
+            assert np.array_equal(q_of(an), ora.get_q()), (rep, name)
+            assert np.array_equal(an.get_E(), ora.calculate_E())
+        if rep == 2:
+            q = 2 * rng.integers(0, 2, N).astype(np.int8) - 1
+            ora.set_q(np.tile(q, (m, 1)))
+            an.set_q(q)
+        elif rep == 4:
+            ora.randomize_spin()
+            an.randomize_spin()
+        assert np.array_equal(q_of(an), ora.get_q()), rep
+
+
 @pytest.mark.parametrize("N,spb,dtype", [(20, 0, np.float32), (100, 0, np.float32), (100, 0, np.float64),
                                          (100, 2, np.float32), (300, 1, np.float32), (1100, 0, np.float32)])
 def test_one_slice_coloring_bit_exact(oracle, rocm, N, spb, dtype):

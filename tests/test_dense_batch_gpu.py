@@ -85,6 +85,21 @@ def test_batch_k_split_gemm_path(rocm, form):
         assert np.array_equal(b.get_E(i), E), i
 
 
+def test_batch_of_short_slices(rocm):
+    """More slices than waves, most so short that one can end before its
+    neighbour is taken from the queue: an odd number of steps, then an even one,
+    equal to the instances annealed alone."""
+    steps = schedule()[:35]
+    probs = [(dense_int_W(N, SEED_BASE + 150 + i), m, 8000 + i)
+             for i, (N, m) in enumerate([(600, 100), (5, 64), (16, 128)] + [(9 + 5 * k, 96) for k in range(30)])]
+    b = batch(rocm, probs, steps[:21])
+    b.anneal(steps[21:], BETA, graph=False)
+    for i, (W, m, seed) in enumerate(probs):
+        q, E = alone(rocm, W, m, seed, steps)
+        assert np.array_equal(b.get_q(i), q), f"instance {i} (N={W.shape[0]}, m={m})"
+        assert np.array_equal(b.get_E(i), E), i
+
+
 def test_autotune_and_schedule_split_do_not_change_results(rocm):
     """Autotuning restores spins, fields and streams; a schedule run as two
     graphs equals one run as a single graph."""
