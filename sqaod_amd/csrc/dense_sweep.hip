@@ -1204,8 +1204,7 @@ template void denseSweepBatch<float>(const SweepArgs<float> *, const uint2 *, in
 template void denseSweepBatch<double>(const SweepArgs<double> *, const uint2 *, int, int *, bool, int, size_t, int,
                                       int, hipStream_t);
 
-/* Whether every block of a launch of fn fits on the device at once. */
-static bool fitsAtOnce(const void *fn, int threads, size_t lds, int nBlocks, int numCUs) {
+bool fitsAtOnce(const void *fn, int threads, size_t lds, int nBlocks, int numCUs) {
     static std::mutex mu;
     static std::map<std::tuple<const void *, int, size_t>, int> perCU;
     std::lock_guard<std::mutex> lock(mu);
@@ -1213,6 +1212,7 @@ static bool fitsAtOnce(const void *fn, int threads, size_t lds, int nBlocks, int
     auto it = perCU.find(key);
     if (it == perCU.end()) {
         int n = 0;
+        HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, threads, lds));
         it = perCU.emplace(key, n).first;
     }

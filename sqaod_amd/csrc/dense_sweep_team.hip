@@ -727,8 +727,17 @@ static int teamTable(int N, int Np, int S, size_t realSize, size_t maxLds) {
 }
 
 int denseSweepTeamSlices(int N, int Np, int m, size_t realSize, int asked, int numCUs, size_t maxLds) {
-    if (asked > 0)
-        return asked <= kTeamMaxSlices && teamTable(N, Np, asked, realSize, maxLds) ? asked : 0;
+    if (asked > 0) {
+        const int tableN = asked <= kTeamMaxSlices ? teamTable(N, Np, asked, realSize, maxLds) : 0;
+        if (tableN == 0)
+            return 0;
+        /* a team takes more LDS than one wave: 256 of them at N=4096 where 512
+         * slices of the one-wave sweep fit */
+        const int nBlocks = divru(m, asked);
+        const void *fn = realSize == 8 ? (const void *)denseSweepTeamKernel<double> : (const void *)denseSweepTeamKernel<float>;
+        const size_t lds = teamLdsBytes(N, Np, tableN, asked, realSize);
+        return nBlocks <= numCUs || fitsAtOnce(fn, kTeamWaves * asked * kWave, lds, nBlocks, numCUs) ? asked : 0;
+    }
     /* as many slices as LDS holds: they read each other's decisions there, in a
      * quarter of the time it takes over device memory (N=1200, m=300: 53.6 us a
      * sweep with three, 55.0 with two, 56.3 with one on twice the blocks there

@@ -316,13 +316,17 @@ void denseSweep(const SweepArgs<real> &args, bool plain, int fieldFormat, int sl
 void launchSweep(void *kernel, int nBlocks, int threads, size_t lds, void **kargs, bool allowDirect, int numCUs,
                  hipStream_t stream);
 
+/* Whether every block of a launch of fn fits on the device at once. */
+bool fitsAtOnce(const void *fn, int threads, size_t lds, int nBlocks, int numCUs);
+
 /* The local-field sweep (float: rows of args.J; double) by a team of four waves
  * per slice, each batch ending at its first flip (dense_sweep_team.hip).
  * args.P: m rows of args.ldP >= teamWordStride(N) words; args.tag: 1 to
  * kTeamTagPeriod, no tag twice without P cleared in between. */
 constexpr uint32_t kTeamTagPeriod = 2047;
 int teamWordStride(int N);
-/* Slices per block (asked: 0 to choose), 0 where the sweep does not fit. */
+/* Slices per block (asked: 0 to choose), 0 where the sweep does not fit: in LDS,
+ * or with all its blocks on the device at once. */
 int denseSweepTeamSlices(int N, int Np, int m, size_t realSize, int asked, int numCUs, size_t maxLds);
 template <class real>
 void denseSweepTeam(const SweepArgs<real> &args, int slicesPerBlock, size_t maxLds, bool allowDirect, int numCUs,

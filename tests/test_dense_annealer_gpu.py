@@ -507,6 +507,26 @@ def test_spins_follow_through_changing_steps(oracle, rocm):
         assert np.array_equal(q_of(an), ora.get_q()), rep
 
 
+@pytest.mark.parametrize("N,m,spb,dtype", [(4096, 300, 1, np.float32), (1024, 600, 2, np.float32),
+                                           (2000, 500, 1, np.float64), (300, 1500, 1, np.float32)])
+def test_more_slices_than_teams_fit(rocm, N, m, spb, dtype):
+    """slices_per_block with more blocks than the team sweep has room for on the
+    chip, which fit with one wave a slice (the last shape: several teams to a
+    CU, more than there are CUs): the same spins as one wave a slice."""
+    W = dense_int_W(N, SEED_BASE + 31).astype(dtype)
+    runs = []
+    for helper in ("on", "off"):
+        an = rocm.dense_graph_annealer(W, dtype=dtype, n_trotters=m, slices_per_block=spb, helper_wave=helper,
+                                       multi_flip="off")
+        an.seed(41)
+        an.prepare()
+        an.randomize_spin()
+        for G in (2.0, 0.5):
+            an.anneal_one_step(G, BETA)
+        runs.append(q_of(an))
+    assert np.array_equal(runs[0], runs[1])
+
+
 @pytest.mark.parametrize("N,spb,dtype", [(20, 0, np.float32), (100, 0, np.float32), (100, 0, np.float64),
                                          (100, 2, np.float32), (300, 1, np.float32), (1100, 0, np.float32)])
 def test_one_slice_coloring_bit_exact(oracle, rocm, N, spb, dtype):
