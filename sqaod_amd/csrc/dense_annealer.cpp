@@ -923,7 +923,8 @@ void DenseGraphAnnealer<real>::annealOneStep(real G, real beta) {
     a.multiBufs = 0;
     if (multi) {
         const int f = fieldFormat_ == fieldFP8 ? fieldF32 : fieldFormat_;
-        a.multiBufs = denseSweepMultiBufs(Np_, S, sizeof(real), plainSweep_, f, dev_->maxLdsPerBlock());
+        a.multiBufs = denseSweepMultiBufs(Np_, S, sizeof(real), plainSweep_, f, dev_->maxLdsPerBlock(), divru(m_, S),
+                                          dev_->numCUs());
         if (a.multiBufs >= 2)
             sweepFormat = f;
     }

@@ -1147,14 +1147,18 @@ size_t denseSweepLdsBytes(int Np, int slicesPerBlock, size_t realSize, bool plai
            waveBytesFor(Np, realSize, plain, fieldFormat, ld8, multiBufs) * slicesPerBlock;
 }
 
-int denseSweepMultiBufs(int Np, int slicesPerBlock, size_t realSize, bool plain, int fieldFormat, size_t maxLds) {
+int denseSweepMultiBufs(int Np, int slicesPerBlock, size_t realSize, bool plain, int fieldFormat, size_t maxLds,
+                        int nBlocks, int numCUs) {
     if (realSize != 4 || plain || fieldFormat == fieldFP8)
         return 0;
     const int rowOps = Np * 4 / (kWave * 16); /* 1 KiB DMA ops per row */
-    for (int b = 4; b >= 2; --b)
-        if ((b - 1) * rowOps <= 63 &&
-            denseSweepLdsBytes(Np, slicesPerBlock, realSize, plain, fieldFormat, 0, b) <= maxLds)
+    for (int b = 4; b >= 2; --b) {
+        const size_t lds = denseSweepLdsBytes(Np, slicesPerBlock, realSize, plain, fieldFormat, 0, b);
+        if ((b - 1) * rowOps <= 63 && lds <= maxLds &&
+            (nBlocks <= numCUs || fitsAtOnce((const void *)denseSweepKernel<float, kModeLocal, true>,
+                                             slicesPerBlock * kWave, lds, nBlocks, numCUs)))
             return b;
+    }
     return 0;
 }
 

@@ -337,9 +337,11 @@ void denseSweepTeam(const SweepArgs<real> &args, int slicesPerBlock, size_t maxL
 size_t denseSweepLdsBytes(int Np, int slicesPerBlock, size_t realSize, bool plain, int fieldFormat = fieldF32,
                           int ld8 = 0, int multiBufs = 0);
 /* Row stage buffers for multi-flip batches that fit beside S slices' regions
- * in maxLds bytes (0: none; at most 4, and (buffers - 1) rows of DMA ops within
- * the 63 outstanding memory operations a wave can count). */
-int denseSweepMultiBufs(int Np, int slicesPerBlock, size_t realSize, bool plain, int fieldFormat, size_t maxLds);
+ * in maxLds bytes and leave all nBlocks blocks on the device at once (0: none;
+ * at most 4, and (buffers - 1) rows of DMA ops within the 63 outstanding memory
+ * operations a wave can count). */
+int denseSweepMultiBufs(int Np, int slicesPerBlock, size_t realSize, bool plain, int fieldFormat, size_t maxLds,
+                        int nBlocks, int numCUs);
 
 /* Many instances in one persistent launch (one wave per (instance, slice)
  * item, taken from a queue in item order; items of one instance must be

@@ -527,6 +527,25 @@ def test_more_slices_than_teams_fit(rocm, N, m, spb, dtype):
     assert np.array_equal(runs[0], runs[1])
 
 
+@pytest.mark.parametrize("N,m,spb,mode", [(4096, 300, 1, "auto"), (1024, 2000, 0, "auto"), (2048, 600, 2, "on")])
+def test_more_slices_than_multi_flip_blocks_fit(rocm, N, m, spb, mode):
+    """The multi-flip sweep's stage buffers give way, to two and then to the
+    single-flip sweep, where with them the blocks would not fit on the chip:
+    the same spins as single-flip sweeps."""
+    W = dense_int_W(N, SEED_BASE + 43)
+    runs = []
+    for multi in (mode, "off"):
+        an = rocm.dense_graph_annealer(W, dtype=np.float32, n_trotters=m, slices_per_block=spb, helper_wave="off",
+                                       multi_flip=multi)
+        an.seed(47)
+        an.prepare()
+        an.randomize_spin()
+        for G in (2.0, 0.5):
+            an.anneal_one_step(G, BETA)
+        runs.append(q_of(an))
+    assert np.array_equal(runs[0], runs[1])
+
+
 @pytest.mark.parametrize("N,spb,dtype", [(20, 0, np.float32), (100, 0, np.float32), (100, 0, np.float64),
                                          (100, 2, np.float32), (300, 1, np.float32), (1100, 0, np.float32)])
 def test_one_slice_coloring_bit_exact(oracle, rocm, N, spb, dtype):
