@@ -39,12 +39,16 @@ struct Error : std::runtime_error {
             SQ_THROW(__VA_ARGS__); \
     } while (0)
 
+/* A reported error is also taken from the thread's last error, where the next
+ * launch's check would find it again. */
 #define HIP_CHECK(expr)                                                                       \
     do {                                                                                      \
         hipError_t e_ = (expr);                                                               \
-        if (e_ != hipSuccess)                                                                 \
+        if (e_ != hipSuccess) {                                                               \
+            (void)hipGetLastError();                                                          \
             ::sqaod_rocm::throwErrorf(__FILE__, __LINE__, "HIP error %d (%s) in %s", (int)e_, \
                                       hipGetErrorString(e_), #expr);                          \
+        }                                                                                     \
     } while (0)
 
 __host__ __device__ inline int divru(int a, int b) { return (a + b - 1) / b; }

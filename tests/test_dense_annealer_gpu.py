@@ -527,6 +527,26 @@ def test_more_slices_than_teams_fit(rocm, N, m, spb, dtype):
     assert np.array_equal(runs[0], runs[1])
 
 
+def test_refused_launch_is_reported_once(rocm):
+    """More slices, one a block, than any sweep has room for: the step's launch
+    is refused with an error, and the next solver's calls do not meet it again."""
+    N, m = 4096, 1100
+    an = rocm.dense_graph_annealer(dense_int_W(N, SEED_BASE + 53), dtype=np.float32, n_trotters=m, slices_per_block=1,
+                                   multi_flip="off")
+    an.seed(1)
+    an.prepare()
+    an.randomize_spin()
+    with pytest.raises(RuntimeError, match="too many blocks"):
+        an.anneal_one_step(1.0, BETA)
+    rocm.dense_graph_bf_searcher(dense_graph_8x8(np.float32), dtype=np.float32).search()
+    other = rocm.dense_graph_annealer(dense_int_W(64, SEED_BASE), dtype=np.float32, n_trotters=4)
+    other.seed(1)
+    other.prepare()
+    other.randomize_spin()
+    other.anneal_one_step(1.0, BETA)
+    other.get_E()
+
+
 @pytest.mark.parametrize("N,m,spb,mode", [(4096, 300, 1, "auto"), (1024, 2000, 0, "auto"), (2048, 600, 2, "on")])
 def test_more_slices_than_multi_flip_blocks_fit(rocm, N, m, spb, mode):
     """The multi-flip sweep's stage buffers give way, to two and then to the
