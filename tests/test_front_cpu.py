@@ -133,3 +133,21 @@ def test_common_helpers():
     assert common.fix_type(np.arange(3), np.float32).dtype == np.float32
     pair = common.fix_type([np.arange(2), [1.5]], np.float64)  # a list: each element fixed
     assert [p.dtype for p in pair] == [np.float64, np.float64] and pair[1].tolist() == [1.5]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("make", [np.triu, np.tril, lambda W: np.triu(W * (np.abs(np.subtract.outer(range(300), range(300))) < 2))],
+                         ids=["upper", "lower", "chain"])
+def test_triangular_energies_take_one_device_call(make, dtype):
+    """W given as one triangle: its energies are not formed on the device only to
+    find that it is not symmetric; they are those of (W + W^T) / 2, in one call."""
+    from sqaod_amd.common import formulas_base
+    rec = Recorder()
+    W = make(np.random.default_rng(5).standard_normal((300, 300)).astype(dtype))
+    x = np.ones((2, 300), np.int8)
+    formulas_base.dense_graph_batch_calculate_E(rec, "c", W, x, dtype)
+    assert [c[0] for c in rec.calls] == ["dense_graph_batch_calculate_E"]
+    assert np.array_equal(rec.calls[0][1][2], (W + W.T) * dtype(0.5))
+    rec.calls.clear()
+    formulas_base.dense_graph_batch_calculate_E(rec, "c", W + W.T, x, dtype)
+    assert [c[0] for c in rec.calls] == ["dense_graph_batch_calculate_E_if_symmetric"]
