@@ -24,7 +24,11 @@ namespace sqaod_rocm {
 
 namespace {
 constexpr unsigned long long kMaxItems = 1ull << 15; /* items per rectangle (each 16 x 2^L pairs) */
+constexpr unsigned long long kMaxX1 = 4096;          /* x1 values per rectangle */
 constexpr unsigned long long kFirstPairs = 64;       /* pairs read back with their number */
+static_assert((2 + 2 * kFirstPairs) * sizeof(unsigned long long) <= Device::HostStage::kBytes &&
+                  kMaxX1 / kBGBFScanBlock * sizeof(double) <= Device::HostStage::kBytes,
+              "both fit in the staging block");
 }  // namespace
 
 template <class real>
@@ -110,8 +114,8 @@ void BipartiteGraphBFSearcher<real>::prepare() {
     T0_ = std::min<unsigned long long>((unsigned long long)tileSize0_, 1ull << N0_);
     plan_ = bgBFPlan(N0_, N1_);
     plan_.sgn = (om_ == optMaximize) ? -1. : 1.;
-    /* rectangles: up to 4096 x1 values times enough high patterns for kMaxItems items */
-    x1Chunk_ = std::min<unsigned long long>(1ull << N1_, 4096);
+    /* rectangles: up to kMaxX1 x1 values times enough high patterns for kMaxItems items */
+    x1Chunk_ = std::min<unsigned long long>(1ull << N1_, kMaxX1);
     const unsigned long long nHigh = 1ull << plan_.nH;
     hChunk_ = std::min<unsigned long long>(nHigh, std::max<unsigned long long>(1, kMaxItems / x1Chunk_) *
                                                       (unsigned long long)kBGBFHighPerBlock);
@@ -120,10 +124,6 @@ void BipartiteGraphBFSearcher<real>::prepare() {
     const unsigned long long items = x1Chunk_ * ((hChunk_ + kBGBFHighPerBlock - 1) / kBGBFHighPerBlock);
     d_x1Min_.allocate(x1Chunk_);
     d_pairs_.allocate(2 + items * 2 * (size_t)plan_.K);
-    h_pairs_.allocate(2 + 2 * kFirstPairs);
-    h_blockMin_.allocate((size_t)((x1Chunk_ + kBGBFScanBlock - 1) / kBGBFScanBlock),
-                         hipHostMallocCoherent | hipHostMallocMapped);
-    HIP_CHECK(hipHostGetDevicePointer((void **)&d_blockMin_, h_blockMin_.ptr, 0));
     setState(solPrepared);
 }
 
@@ -140,9 +140,12 @@ bool BipartiteGraphBFSearcher<real>::searchRange(unsigned long long *curX0, unsi
         a.x1b = x1Next_;
         a.nX1 = std::min(x1Chunk_, x1max - x1Next_);
         hipStream_t st = dev_->stream();
-        bgBFScan<real>(a, d_b0_.ptr, d_b1_.ptr, d_W_.ptr, d_x1Min_.ptr, d_blockMin_, d_pairs_.ptr, st);
+        Device::HostStage stage(*dev_); /* the scan's minima, then the pairs */
+        bgBFScan<real>(a, d_b0_.ptr, d_b1_.ptr, d_W_.ptr, d_x1Min_.ptr, reinterpret_cast<real *>(stage.device()),
+                       d_pairs_.ptr, st);
         HIP_CHECK(hipStreamSynchronize(st));
-        const real rmin = *std::min_element(h_blockMin_.ptr, h_blockMin_.ptr + bgBFScanBlocks(a));
+        const real *blockMin = reinterpret_cast<const real *>(stage.host());
+        const real rmin = *std::min_element(blockMin, blockMin + bgBFScanBlocks(a));
         if (rmin <= Emin_) {
             if (rmin < Emin_) {
                 Emin_ = rmin;
@@ -150,12 +153,13 @@ bool BipartiteGraphBFSearcher<real>::searchRange(unsigned long long *curX0, unsi
             }
             bgBFSelect<real>(a, d_b0_.ptr, d_b1_.ptr, d_W_.ptr, d_x1Min_.ptr, rmin, d_pairs_.ptr + 2, d_pairs_.ptr,
                              st);
-            const size_t room = std::min<size_t>(h_pairs_.n, d_pairs_.n);
-            HIP_CHECK(hipMemcpyAsync(h_pairs_.ptr, d_pairs_.ptr, room * sizeof(unsigned long long),
+            unsigned long long *const first = reinterpret_cast<unsigned long long *>(stage.host());
+            const size_t room = std::min<size_t>(2 + 2 * kFirstPairs, d_pairs_.n);
+            HIP_CHECK(hipMemcpyAsync(first, d_pairs_.ptr, room * sizeof(unsigned long long),
                                      hipMemcpyDeviceToHost, st));
             HIP_CHECK(hipStreamSynchronize(st));
-            const size_t n = (size_t)h_pairs_.ptr[0];
-            const unsigned long long *pairs = h_pairs_.ptr + 2;
+            const size_t n = (size_t)first[0];
+            const unsigned long long *pairs = first + 2;
             std::vector<unsigned long long> all;
             if (2 + 2 * n > room) {
                 all.resize(2 * n);
@@ -175,6 +179,7 @@ bool BipartiteGraphBFSearcher<real>::searchRange(unsigned long long *curX0, unsi
             for (size_t k = 0; k < cand.size() && k < K; ++k)
                 list_.push_back(cand[k].second);
         }
+        stage.done();
         /* next rectangle: x1 chunks inside, high-pattern chunks outside */
         x1Next_ += a.nX1;
         if (x1Next_ >= x1max) {

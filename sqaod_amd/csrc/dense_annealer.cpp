@@ -103,6 +103,7 @@ void SolverState::throwErrorIfQNotSet() const {
 }
 
 Device::Device(int devno) : devno_(devno) {
+    stages_.reserve(kKeptStages); /* giving one back then cannot fail */
     int n = 0;
     HIP_CHECK(hipGetDeviceCount(&n));
     SQ_THROW_IF(devno < 0 || devno >= n, "device %d not available (%d devices)", devno, n);
@@ -139,6 +140,38 @@ Device::~Device() {
     (void)hipSetDevice(devno_);
     (void)hipStreamSynchronize(stream_);
     (void)hipStreamDestroy(stream_);
+    for (unsigned char *p : stages_)
+        (void)hipHostFree(p);
+}
+
+Device::HostStage::HostStage(Device &dev) : dev_(dev) {
+    {
+        std::lock_guard<std::mutex> lock(dev.stagesMu_);
+        if (!dev.stages_.empty()) {
+            host_ = dev.stages_.back();
+            dev.stages_.pop_back();
+        }
+    }
+    if (!host_)
+        HIP_CHECK(hipHostMalloc((void **)&host_, kBytes, hipHostMallocCoherent | hipHostMallocMapped));
+    const hipError_t e = hipHostGetDevicePointer((void **)&device_, host_, 0);
+    if (e != hipSuccess) {
+        (void)hipHostFree(host_);
+        HIP_CHECK(e);
+    }
+}
+
+Device::HostStage::~HostStage() {
+    if (!done_)
+        (void)hipStreamSynchronize(dev_.stream_);
+    {
+        std::lock_guard<std::mutex> lock(dev_.stagesMu_);
+        if (dev_.stages_.size() < kKeptStages) {
+            dev_.stages_.push_back(host_);
+            return;
+        }
+    }
+    (void)hipHostFree(host_);
 }
 
 void Device::makeCurrent() const { HIP_CHECK(hipSetDevice(devno_)); }

@@ -62,7 +62,32 @@ public:
      * process: then no sweep of another stream can run beside its sweeps. */
     bool soleSweeper();
 
+    /* A block of pinned host memory that kernels and copies of this Device's
+     * stream may write, for one call's use: kept by the Device (up to
+     * kKeptStages of them), since allocating one takes as long as a small
+     * search.  Any thread may take one; before it goes back the stream is
+     * synchronised unless the holder says that its work is done. */
+    class HostStage {
+    public:
+        static constexpr size_t kBytes = 4096;
+        explicit HostStage(Device &dev);
+        ~HostStage();
+        HostStage(const HostStage &) = delete;
+        HostStage &operator=(const HostStage &) = delete;
+        unsigned char *host() const { return host_; }
+        unsigned char *device() const { return device_; } /* the same as kernels see it */
+        void done() { done_ = true; }
+
+    private:
+        Device &dev_;
+        unsigned char *host_ = nullptr, *device_ = nullptr;
+        bool done_ = false;
+    };
+
 private:
+    static constexpr size_t kKeptStages = 8;
+    std::mutex stagesMu_;
+    std::vector<unsigned char *> stages_; /* free ones */
     int devno_;
     hipStream_t stream_;
     bool sweeper_ = false;
@@ -485,9 +510,6 @@ private:
     std::vector<real> E_;
     DevBuf<real> d_b0_, d_b1_, d_W_, d_x1Min_;
     DevBuf<unsigned long long> d_pairs_; /* the number of pairs (2 words), then the pairs */
-    PinnedBuf<real> h_blockMin_;
-    PinnedBuf<unsigned long long> h_pairs_;
-    real *d_blockMin_ = nullptr; /* h_blockMin_ as the device sees it */
 };
 
 /* ------------------------------------------------------------------ */

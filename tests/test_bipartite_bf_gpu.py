@@ -96,6 +96,29 @@ def test_errors(rocm):
         s.prepare()
 
 
+def test_many_searchers_on_several_threads(rocm):
+    """The minima and first pairs of a rectangle come back through staging memory
+    of the device: more searchers than it keeps blocks for, on several threads
+    at once, each find what they find alone."""
+    from concurrent.futures import ThreadPoolExecutor
+    rng = np.random.default_rng(SEED_BASE + 77)
+    problems = [tuple(rng.integers(-3, 4, s).astype(np.float32) for s in (n0, n1, (n1, n0)))
+                for n0, n1 in [(3 + k % 10, 2 + (3 * k) % 13) for k in range(24)]]
+
+    def search(p):
+        s = rocm.bipartite_graph_bf_searcher(*p, dtype=np.float32)
+        for _ in range(3):
+            s.search()
+        return s, s.get_E(), s.get_x()
+
+    alone = [search(p) for p in problems]
+    with ThreadPoolExecutor(12) as pool:
+        together = list(pool.map(search, problems))
+    for (_, E0, x0), (_, E1, x1) in zip(alone, together):
+        assert np.array_equal(E0, E1) and len(x0) == len(x1)
+        assert all(np.array_equal(a, b) for p, q in zip(x0, x1) for a, b in zip(p, q))
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("N0,N1", [(1, 1), (63, 1), (11, 5), (4, 12), (20, 1), (18, 13)])
 def test_real_weights_take_the_least_over_x0(rocm, dtype, N0, N1):
