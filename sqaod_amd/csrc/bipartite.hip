@@ -38,8 +38,15 @@ constexpr int kSites = 8; /* of a block of all phases */
  * at 1024 x 64 spins, 6.6 against 2 x 4.8 at 8192 x 64, 9.8 against 2 x 4.9
  * at 4096 x 256, 16.2 against 2 x 7.2 at 8192 x 256. */
 constexpr long long kMaxFusedSpins = 1 << 20;
-/* It holds four bytes a slice in LDS. */
-constexpr int kMaxFusedSlices = 65536 / 4;
+/* A block walks all slices of its 8 sites, 128 at a time, however few blocks
+ * there are, so it loses to launches over slices and sites once the slices are
+ * many: two for an even number, three for an odd one.  A step (us, one launch a
+ * side / by phase, N0 = N1; float): N = 64: 14.9 / 19.1 with m = 192, 20.0 /
+ * 19.0 with 256, 73 / 19 with 2048, 19.7 / 27.3 with 321, 25.4 / 28.2 with 511;
+ * N = 1024: 21.3 / 22.7, 27.5 / 23.8, (1024 slices) 65 / 47, 28.7 / 31.4,
+ * 36.6 / 34.8; double N = 64: 15.1 / 16.6, 19.5 / 18.8, 74 / 18, 20.0 / 21.6,
+ * 25.1 / 21.7. */
+constexpr int kMaxFusedSlicesEven = 192, kMaxFusedSlicesOdd = 320;
 
 template <class real>
 __device__ __forceinline__ real expNeg(real x);
@@ -175,7 +182,7 @@ __global__ __launch_bounds__(kMaxThreads) void bgFlipsKernel(BGFlipArgs<real> a)
 template <class real>
 bool bipartiteFlips(const BGFlipArgs<real> &a, hipStream_t stream) {
     SQ_THROW_IF(a.N <= 0 || a.m <= 0 || a.Nw * 32 < a.N, "bipartite flips: bad row of %d spins in %d words", a.N, a.Nw);
-    if (a.sa || a.m > kMaxFusedSlices || (long long)a.N * a.m > kMaxFusedSpins)
+    if (a.sa || a.m > (a.m % 2 ? kMaxFusedSlicesOdd : kMaxFusedSlicesEven) || (long long)a.N * a.m > kMaxFusedSpins)
         return false;
     const int threads = std::min(roundUp(a.m * kSites, kWave), kMaxThreads);
     bgFlipsKernel<real><<<divru(a.N, kSites), threads, (size_t)a.m * 4, stream>>>(a);

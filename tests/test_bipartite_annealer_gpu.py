@@ -94,8 +94,12 @@ def test_bit_exact_float64_coloring(oracle, rocm):
     (7, 9, 2),           # part of a byte, one byte and a bit; both neighbours the same slice
     (8, 33, 3),
     (65, 1, 129),        # more spins than a block has threads
-    (3, 2, 16384),       # the most slices of one launch for all phases
-    (3, 2, 16385),       # phase by phase, odd
+    (70, 17, 192),       # the most slices, even and odd, of one launch for all phases
+    (9, 70, 194),        # phase by phase
+    (70, 17, 319),
+    (9, 70, 321),
+    (3, 2, 16384),
+    (3, 2, 16385),
     (16384, 2, 64),      # the most spins of one launch
     (16385, 2, 64),      # phase by phase on one side only
 ])
