@@ -224,8 +224,10 @@ constexpr int kQfTile = 32; /* rows of V, rows of A and columns of both in a til
  * zero, which a product with zero does not give: such an A (or a stored sum
  * that is not finite) is flagged and quadFormKernel evaluates the outputs term
  * by term.  So it does where nu nv <= kQfDirect, in one launch: a whole call on
- * 64 x 64 takes 52 us for one vector and 86 us for 1000 that way, which the two
- * launches do not beat, and on 96 x 96 and 100 vectors 72 us against 68 us.
+ * 100 pairs of float vectors takes 43 us against 45 for 20 x 20 that way, 50
+ * against 51 for 40 x 50, and 46 against 44 for 64 x 64.  (All pairs of many
+ * vectors would gain by the two launches sooner: 100 x 100 pairs of 20 x 20,
+ * 75 against 68 us.)
  * Measured, 1000 x 1000 floats and 500 vectors: 39.9 + 5.7 us against 702 us
  * for the one-launch form; bound by the round trip of a tile's loads (the
  * products alone take 14 us at the 71 TFLOP/s a large FP64 product reaches). */
@@ -322,9 +324,11 @@ __global__ __launch_bounds__(kQfThreads) void quadFormKernel(QuadFormArgs<real> 
     const int8_t *u = a.U + (size_t)bu * a.nu;
     const int8_t *v = a.V + (size_t)bv * a.nv;
     int direct = work == nullptr;
-    for (int f = threadIdx.x; f < nFlags; f += kQfThreads)
-        direct |= flags[f];
-    direct = __syncthreads_or(direct);
+    if (!direct) {
+        for (int f = threadIdx.x; f < nFlags; f += kQfThreads)
+            direct |= flags[f];
+        direct = __syncthreads_or(direct);
+    }
     double s = 0.;
     if (direct) {
         for (int i = threadIdx.x; i < a.nu; i += kQfThreads) {

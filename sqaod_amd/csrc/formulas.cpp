@@ -18,6 +18,10 @@
 
 namespace sqaod_rocm {
 
+namespace {
+constexpr size_t kPackedBytes = 256 << 10; /* vectors copied together up to here: they are copied twice on the host */
+}  // namespace
+
 template <class real>
 void Formulas<real>::assignDevice(Device &dev) {
     SQ_THROW_IF(dev_ != nullptr && dev_ != &dev, "Device assigned more than once.");
@@ -38,45 +42,59 @@ void Formulas<real>::run(QuadFormArgs<real> a, const real *A, size_t nA, const r
                          real *E, int nOut, bool *symmetric) {
     Device &dev = device();
     hipStream_t st = dev.stream();
-    DevBuf<real> dA, d0, d1, dE;
-    DevBuf<int8_t> dU, dV;
-    dA.allocate(nA);
-    dE.allocate((size_t)nOut);
-    dU.allocate(nU);
-    HIP_CHECK(hipMemcpyAsync(dA.ptr, A, nA * sizeof(real), hipMemcpyHostToDevice, st));
-    HIP_CHECK(hipMemcpyAsync(dU.ptr, U, nU, hipMemcpyHostToDevice, st));
-    a.A = dA.ptr;
-    a.U = dU.ptr;
-    a.V = dU.ptr;
-    if (V != U) {
-        dV.allocate(nV);
-        HIP_CHECK(hipMemcpyAsync(dV.ptr, V, nV, hipMemcpyHostToDevice, st));
-        a.V = dV.ptr;
+    /* One allocation for everything, and one copy for the vectors while they are
+     * small: with an allocation and a copy for each, the second launch of the
+     * two-launch form made bipartite calls slower than the one-launch form,
+     * although its kernels are faster (10 pairs of 64 + 65 floats, whole calls:
+     * 83 us against 62; now 46). */
+    const size_t workBytes = quadFormWorkBytes(a.nu, a.nv, a.nV, a.twoD != 0);
+    size_t end = 0;
+    auto place = [&](size_t bytes) {
+        const size_t at = end;
+        end = (end + bytes + 63) / 64 * 64;
+        return at;
+    };
+    struct Part {
+        const void *src;
+        size_t bytes, at;
+    };
+    const size_t oA = place(nA * sizeof(real)), oParts = end;
+    const Part parts[] = {{U, nU, place(nU)},
+                          {V, V != U ? nV : 0, V != U ? place(nV) : 0},
+                          {lin0, lin0 ? n0 * sizeof(real) : 0, place(lin0 ? n0 * sizeof(real) : 0)},
+                          {lin1, lin1 ? n1 * sizeof(real) : 0, place(lin1 ? n1 * sizeof(real) : 0)}};
+    const size_t partsBytes = end - oParts;
+    const size_t oWork = place(workBytes), oFlag = place(sizeof(int)), oE = place((size_t)nOut * sizeof(real));
+    DevBuf<unsigned char> mem;
+    mem.allocate(end);
+    unsigned char *const d = mem.ptr;
+    HIP_CHECK(hipMemcpyAsync(d + oA, A, nA * sizeof(real), hipMemcpyHostToDevice, st));
+    std::vector<unsigned char> packed;
+    if (parts[1].bytes + parts[2].bytes + parts[3].bytes != 0 && partsBytes <= kPackedBytes) {
+        packed.resize(partsBytes);
+        for (const Part &p : parts)
+            if (p.bytes)
+                memcpy(packed.data() + (p.at - oParts), p.src, p.bytes);
+        HIP_CHECK(hipMemcpyAsync(d + oParts, packed.data(), partsBytes, hipMemcpyHostToDevice, st));
+    } else {
+        for (const Part &p : parts)
+            if (p.bytes)
+                HIP_CHECK(hipMemcpyAsync(d + p.at, p.src, p.bytes, hipMemcpyHostToDevice, st));
     }
-    a.lin0 = a.lin1 = nullptr;
-    if (lin0) {
-        d0.allocate(n0);
-        HIP_CHECK(hipMemcpyAsync(d0.ptr, lin0, n0 * sizeof(real), hipMemcpyHostToDevice, st));
-        a.lin0 = d0.ptr;
-    }
-    if (lin1) {
-        d1.allocate(n1);
-        HIP_CHECK(hipMemcpyAsync(d1.ptr, lin1, n1 * sizeof(real), hipMemcpyHostToDevice, st));
-        a.lin1 = d1.ptr;
-    }
-    a.E = dE.ptr;
-    DevBuf<int> dAsymmetric;
+    a.A = reinterpret_cast<real *>(d + oA);
+    a.U = reinterpret_cast<int8_t *>(d + parts[0].at);
+    a.V = V != U ? reinterpret_cast<int8_t *>(d + parts[1].at) : a.U;
+    a.lin0 = lin0 ? reinterpret_cast<real *>(d + parts[2].at) : nullptr;
+    a.lin1 = lin1 ? reinterpret_cast<real *>(d + parts[3].at) : nullptr;
+    a.E = reinterpret_cast<real *>(d + oE);
+    int *const dAsymmetric = reinterpret_cast<int *>(d + oFlag);
     int asymmetric = 0;
-    if (symmetric) {
-        dAsymmetric.allocate(1);
-        symmetricCheck<real>(dA.ptr, a.nu, dAsymmetric.ptr, st);
-    }
-    DevBuf<unsigned char> dWork;
-    dWork.allocate(quadFormWorkBytes(a.nu, a.nv, a.nV, a.twoD != 0));
-    quadForm<real>(a, nOut, dWork.ptr, dWork.n, st);
-    HIP_CHECK(hipMemcpyAsync(E, dE.ptr, (size_t)nOut * sizeof(real), hipMemcpyDeviceToHost, st));
     if (symmetric)
-        HIP_CHECK(hipMemcpyAsync(&asymmetric, dAsymmetric.ptr, sizeof(int), hipMemcpyDeviceToHost, st));
+        symmetricCheck<real>(a.A, a.nu, dAsymmetric, st);
+    quadForm<real>(a, nOut, d + oWork, workBytes, st);
+    HIP_CHECK(hipMemcpyAsync(E, a.E, (size_t)nOut * sizeof(real), hipMemcpyDeviceToHost, st));
+    if (symmetric)
+        HIP_CHECK(hipMemcpyAsync(&asymmetric, dAsymmetric, sizeof(int), hipMemcpyDeviceToHost, st));
     dev.synchronize();
     if (symmetric)
         *symmetric = !asymmetric;

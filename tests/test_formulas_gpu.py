@@ -170,6 +170,23 @@ def test_bipartite_energy_tiles(F, dtype, N0, N1, B0, B1):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_bipartite_energies_of_long_batches(F, dtype):
+    """The vectors of a call go to the device in one copy up to 256 KiB and one
+    by one above: 140 pairs of 950 + 1000 elements are more, 10 of them less.
+    Integer values: sums exact."""
+    rng = np.random.default_rng(SEED_BASE + 83)
+    N0, N1, B = 950, 1000, 140
+    b0, b1, W = (rng.integers(-8, 9, s).astype(dtype) for s in (N0, N1, (N1, N0)))
+    x0, x1 = (rng.integers(0, 2, (B, n)).astype(np.int8) for n in (N0, N1))
+    d0, d1 = x0.astype(np.float64), x1.astype(np.float64)
+    exact = d1 @ W.astype(np.float64) @ d0.T + (d0 @ b0)[None, :] + (d1 @ b1)[:, None]
+    for n in (B, 10):
+        assert np.array_equal(F.bipartite_graph_batch_calculate_E_2d(b0, b1, W, x0[:n], x1[:n], dtype), exact[:n, :n])
+        assert np.array_equal(F.bipartite_graph_batch_calculate_E(b0, b1, W, x0[:n], x1[:n], dtype),
+                              np.diag(exact)[:n])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("N", [255, 256, 257, 288, 300])  # the host's check, then the device's by tiles of 32
 def test_dense_energy_of_unsymmetric_matrices(F, dtype, N):
     """What counts as symmetric does not depend on where W is compared: one
