@@ -632,11 +632,7 @@ void DenseGraphAnnealer<real>::prepare() {
     d_D_.allocate(mN);
     HIP_CHECK(hipMemsetAsync(d_Q_.ptr, 0, d_Q_.bytes(), dev_->stream()));
     HIP_CHECK(hipMemsetAsync(d_D_.ptr, 0, d_D_.bytes(), dev_->stream()));
-    ldP_ = teamWordStride(N_);
-    d_P_.allocate((size_t)m_ * ldP_);
-    HIP_CHECK(hipMemsetAsync(d_P_.ptr, 0, d_P_.bytes(), dev_->stream()));
     tag_ = 0;
-    teamTag_ = 0;
     d_E_.allocate((size_t)m_);
     ensureEnergyPlanes();
     d_spinDot_.allocate(1);
@@ -837,13 +833,31 @@ SweepArgs<real> DenseGraphAnnealer<real>::makeSweepArgs(real G, real beta) {
     a.D = d_D_.ptr;
     reserveTags(1);
     a.tag = ++tag_;
-    a.P = d_P_.ptr;
-    a.ldP = ldP_;
     a.abortFlag = d_abort_.ptr;
     a.abortHost = d_abortHost_;
     a.counters = d_counters_.ptr;
     a.spinLimit = spinLimit_;
     return a;
+}
+
+template <class real>
+void DenseGraphAnnealer<real>::takeTeamWords(SweepArgs<real> &a) {
+    /* made by the first team sweep (instances of a batch never run one) and kept
+     * through prepare(): their tags count the team's sweeps alone, and other
+     * kernels may run any number of sweeps in between without touching them */
+    const int ld = teamWordStride(N_);
+    if (ld != ldP_ || d_P_.n != (size_t)m_ * ld) {
+        d_P_.allocate((size_t)m_ * ld);
+        ldP_ = ld;
+        teamTag_ = kTeamTagPeriod;
+    }
+    if (teamTag_ == kTeamTagPeriod) {
+        HIP_CHECK(hipMemsetAsync(d_P_.ptr, 0, d_P_.bytes(), dev_->stream()));
+        teamTag_ = 0;
+    }
+    a.P = d_P_.ptr;
+    a.ldP = ldP_;
+    a.tag = ++teamTag_;
 }
 
 template <class real>
@@ -966,13 +980,7 @@ void DenseGraphAnnealer<real>::annealOneStep(real G, real beta) {
     if (profile_)
         phaseBegin(2, pe);
     if (teamS > 0 && a.multiBufs < 2) {
-        /* its words' tags count the team's sweeps alone: other kernels may run any
-         * number of sweeps in between without touching the words */
-        if (teamTag_ == kTeamTagPeriod) {
-            teamTag_ = 0;
-            HIP_CHECK(hipMemsetAsync(d_P_.ptr, 0, d_P_.bytes(), dev_->stream()));
-        }
-        a.tag = ++teamTag_;
+        takeTeamWords(a);
         denseSweepTeam<real>(a, teamS, dev_->maxLdsPerBlock(), direct, dev_->numCUs(), dev_->stream());
     } else {
         denseSweep<real>(a, plainSweep_, sweepFormat, S, direct, dev_->numCUs(), dev_->stream());

@@ -238,6 +238,7 @@ private:
     void allocateProblem(int N);
     void refreshFields(bool always = false); /* always: also when the plain sweep needs no fields */
     void annealOneStepNaive(real G, real beta);
+    void takeTeamWords(SweepArgs<real> &a); /* the words and tag of a team sweep */
     void seedWorkerGenerators(); /* d_mt_[w] = MT19937 seeded seed_ + 17 w, w < nWorkers_ */
     void traceSystemE(real G, real beta);
     void generateAttempts();

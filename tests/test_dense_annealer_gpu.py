@@ -599,6 +599,27 @@ def test_team_sweep_after_a_tag_period_of_others(oracle, rocm):
             assert np.array_equal(q_of(an), ora.get_q()), k
 
 
+def test_team_words_follow_the_number_of_slices(rocm):
+    """The published words are kept through prepare() and made anew where the
+    slices' number or length changes (the first change leaves their total as
+    it was): the same spins as one wave a slice."""
+    runs = []
+    for helper in ("on", "off"):
+        an = rocm.dense_graph_annealer(dense_int_W(100, SEED_BASE + 59), dtype=np.float32, helper_wave=helper)
+        out = []
+        for N, m in [(100, 8), (100, 8), (1500, 4), (100, 5), (600, 8), (100, 8)]:
+            an.set_qubo(dense_int_W(N, SEED_BASE + 59))
+            an.set_preferences(n_trotters=m)
+            an.seed(3)
+            an.prepare()
+            an.randomize_spin()
+            for G in (3.0, 0.5, 0.1):
+                an.anneal_one_step(G, BETA)
+            out.append(q_of(an))
+        runs.append(out)
+    assert all(np.array_equal(a, b) for a, b in zip(*runs))
+
+
 def test_team_sweep_past_its_tag_period(oracle, rocm):
     """More sweeps than the published words have tags (2047)."""
     N, m = 24, 4
