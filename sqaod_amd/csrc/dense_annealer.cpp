@@ -955,7 +955,10 @@ void DenseGraphAnnealer<real>::annealOneStep(real G, real beta) {
     /* the team sweep where it fits; the fp8 form's runs on the float copy of J'
      * (a.J): its row updates add the same values, -+2 J'[x][s], exactly */
     int teamS = 0;
-    if (helperWave_ && !plainSweep_)
+    /* (float: not at a negative temperature, where exp(-dE beta) may exceed the
+     * uniform of 1 that its least accepted exponent has no value for) */
+    const bool positive = sizeof(real) == 8 || !((a.sa ? a.invKT : a.beta) < real(0.));
+    if (helperWave_ && !plainSweep_ && positive)
         teamS = denseSweepTeamSlices(N_, Np_, m_, sizeof(real), slicesPerBlock_, dev_->numCUs(), dev_->maxLdsPerBlock());
     /* multi-flip batches where LDS allows (float local-field sweeps; the fp8
      * form's on the float copy of J' as well).  "auto" takes them in the first

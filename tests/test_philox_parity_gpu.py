@@ -260,3 +260,23 @@ def test_serving_poisson_mix_against_oracle(oracle, rocm):
         else:
             q0, q1 = ora.get_q()
             assert np.array_equal(r["x0"], (q0 + 1) // 2) and np.array_equal(r["x1"], (q1 + 1) // 2), f"job {i}"
+
+
+@pytest.mark.parametrize("algo", ["sa_naive", "coloring"])
+@pytest.mark.parametrize("seed", [171, 1201, 1337, 3094, 3651, 3677])
+def test_uniform_of_one_at_a_negative_temperature(oracle, rocm, seed, algo):
+    """One of the first two sweeps' uniforms rounds to 1 with these seeds: at
+    kT < 0, or G and beta < 0, an attempt that raises the energy is accepted
+    even there, since exp(-dE / kT) exceeds 1, and one that lowers it is not."""
+    N, m = 1000, 32
+    W = dense_int_W(N, SEED_BASE + 61)
+    assert max(oracle.philox_attempts(seed, s, N, m, np.float32)[1].max() for s in (1, 2)) == 1.0
+    ora = oracle_dense(oracle, W, m, seed, algo=algo)
+    an = rocm.dense_graph_annealer(W, dtype=np.float32, n_trotters=m, algorithm=algo)
+    an.seed(seed)
+    an.prepare()
+    an.randomize_spin()
+    for _ in range(2):
+        an.anneal_one_step(-5.0, -1.0)
+        ora.anneal_one_step(-5.0, -1.0)
+        assert np.array_equal(np.stack(an.get_q()), ora.get_q())
