@@ -216,6 +216,24 @@ def test_large_instance_runs(rocm, oracle):
     assert cnt["flips"] > 0 and cnt["batches"] > 0
 
 
+@pytest.mark.parametrize("N,m,spb,algo", [(1, 3, 1, "coloring"), (37, 3, 2, "coloring"), (63, 5, 4, "coloring"),
+                                          (257, 6, 2, "coloring"), (1025, 3, 1, "coloring"),
+                                          (200, 5, 4, "sa_naive")])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_one_wave_sweep_bit_exact(oracle, rocm, N, m, spb, algo, dtype):
+    """The single-flip kernel of one wave a slice, which runs where teams do not
+    fit, at the shapes of the team sweep's own test."""
+    W = dense_int_W(N, SEED_BASE + 7 * N + m)
+    ora, an = make_pair(oracle, rocm, W, m, seed=11 + N, algo=algo, dtype=dtype, multi_flip="off",
+                        helper_wave="off", slices_per_block=spb)
+    for G in (np.geomspace(20.0, 0.05, 30) if algo == "sa_naive" else schedule()[:160:5]):
+        beta = 0.0 if algo == "sa_naive" else BETA
+        ora.anneal_one_step(G, beta)
+        an.anneal_one_step(G, beta)
+        assert np.array_equal(q_of(an), ora.get_q())
+    assert np.array_equal(an.get_E(), ora.calculate_E())
+
+
 @pytest.mark.parametrize("form", ["fp32", "bf16x2", "fp8"])
 def test_largest_lds_resident_n_bit_exact(oracle, rocm, form):
     """N = 11520, the largest padded N whose float local-field sweep fits one
@@ -368,10 +386,9 @@ def test_multi_flip_engages_and_matches_single_flip(rocm, N, m):
                                            (1000, 16, "bf16x2", "coloring"), (96, 1, "fp32", "sa_naive"),
                                            (4096, 8, "fp32", "coloring"), (6000, 3, "bf16x2", "coloring")])
 def test_helper_wave_bit_exact(oracle, rocm, N, m, form, algo):
-    """helper_wave=on (the default): a second wave per slice adds the last
-    flip's J row to the LDS fields while the sweeping wave runs the next
-    batch's neighbour phase, the next row streaming into the other stage
-    buffer; the sweeping wave waits for it before reading a field.  With
+    """helper_wave=on (the default): a team of four waves per slice sweeps it,
+    one deciding, one adding the last flip's J row to the LDS fields, one
+    preparing the attempts ahead, one reading the neighbours' decisions.  With
     multi_flip=off every sweep runs that kernel, and the trajectory is still
     the serial CPU annealer's, bit for bit."""
     W = dense_int_W(N, SEED_BASE + 5 * N + m)
@@ -392,8 +409,8 @@ def test_helper_wave_bit_exact(oracle, rocm, N, m, form, algo):
 
 
 def test_helper_wave_on_off_same_sweep(rocm):
-    """The helper wave changes who adds a row to the fields, not the sweep:
-    the same spins, flips and energies with it on and off (float normal W, so
+    """The team changes who does what, not the sweep: one wave a slice commits
+    the same spins, flips and energies (float normal W, so
     the fields carry rounding that any change of operation order would
     show).  Batch counts are not compared: where a batch ends depends on how
     far the neighbour slices have got, which is timing."""
@@ -412,14 +429,17 @@ def test_helper_wave_on_off_same_sweep(rocm):
     assert np.array_equal(runs["off"][2], runs["on"][2])
 
 
-@pytest.mark.parametrize("spb", [2, 4])
-def test_helper_wave_with_several_slices_per_block(oracle, rocm, spb):
-    """The helper wave needs one slice per workgroup: with slices_per_block
-    2 or 4 and helper_wave=on the sweep runs the one-wave kernel, still the
-    serial CPU annealer's trajectory."""
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("helper", ["on", "off"])
+@pytest.mark.parametrize("spb", [1, 2, 4])
+def test_helper_wave_with_several_slices_per_block(oracle, rocm, spb, helper, dtype):
+    """Several slices of a workgroup, each by a team or, with helper_wave=off, by
+    one wave (in single-flip batches), with a last workgroup that
+    is not full: the serial CPU annealer's trajectory."""
     N, m = 300, 7
     W = dense_int_W(N, SEED_BASE + 17 * spb)
-    ora, an = make_pair(oracle, rocm, W, m, seed=61 + spb, slices_per_block=spb, helper_wave="on")
+    ora, an = make_pair(oracle, rocm, W, m, seed=61 + spb, dtype=dtype, slices_per_block=spb, helper_wave=helper,
+                        **({} if helper == "on" else {"multi_flip": "off"}))
     assert int(an.get_preferences()["slices_per_block"]) == spb
     for k, G in enumerate(schedule()[:30]):
         ora.anneal_one_step(G, BETA)
@@ -429,9 +449,9 @@ def test_helper_wave_with_several_slices_per_block(oracle, rocm, spb):
 
 
 def test_helper_wave_near_the_lds_limit(oracle, rocm):
-    """N = 8192: fields, two row stage buffers, h and the pending table fill
-    most of a workgroup's 160 KiB of LDS, and the helper-wave kernel still
-    runs the serial CPU annealer's trajectory."""
+    """N = 8192: fields, two row stage buffers, h and the tables by site (fewer
+    slots than sites) fill most of a workgroup's 160 KiB of LDS, and the team
+    sweep still runs the serial CPU annealer's trajectory."""
     N, m = 8192, 2
     W = dense_int_W(N, SEED_BASE + 8192)
     ora, an = make_pair(oracle, rocm, W, m, seed=73, multi_flip="off", helper_wave="on")

@@ -72,10 +72,10 @@ def test_batch_field_forms(rocm, form):
 
 @pytest.mark.parametrize("form", ["fp32", "bf16x2"])
 def test_batch_k_split_gemm_path(rocm, form):
-    """An instance of 2500 sites (2560 padded, a k-range above 2048) takes the
-    grouped field GEMM's k-split path (the block's four waves share the
-    k-range and add their partial tiles in LDS) beside one that takes the
-    column split; both end equal to the instances annealed alone."""
+    """An instance of 2500 sites (2560 padded, a k-range of 20 super-blocks of
+    128, five to each of a block's four waves) and one of 300 (512 padded: one
+    to a wave) in one grouped field GEMM; both end equal to the instances
+    annealed alone."""
     steps = schedule()[:6]
     probs = [(dense_normal_W(2500, SEED_BASE + 140), 4, 7001), (dense_int_W(300, SEED_BASE + 141), 3, 7002)]
     b = batch(rocm, probs, steps, field_precision=form)
