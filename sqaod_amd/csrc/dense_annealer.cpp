@@ -958,7 +958,9 @@ void DenseGraphAnnealer<real>::annealOneStep(real G, real beta) {
     /* (float: not at a negative temperature, where exp(-dE beta) may exceed the
      * uniform of 1 that its least accepted exponent has no value for) */
     const bool positive = sizeof(real) == 8 || !((a.sa ? a.invKT : a.beta) < real(0.));
-    if (helperWave_ && !plainSweep_ && positive)
+    /* (nor for one slice that is its own neighbour: it keeps no words in LDS,
+     * where a neighbour of the same block is looked for) */
+    if (helperWave_ && !plainSweep_ && positive && (m_ > 1 || a.sa))
         teamS = denseSweepTeamSlices(N_, Np_, m_, sizeof(real), slicesPerBlock_, dev_->numCUs(), dev_->maxLdsPerBlock());
     /* multi-flip batches where LDS allows (float local-field sweeps; the fp8
      * form's on the float copy of J' as well).  "auto" takes them in the first

@@ -693,11 +693,8 @@ __global__ __launch_bounds__(kTeamWaves *kTeamMaxSlices *kWave) void denseSweepT
         if (a.sa)
             return;
         const Neighbours nb = neighboursOf(y, a.m);
-        /* one slice a block keeps no words of its own: with m = 1, where it is its
-         * own neighbour, it reads them from memory as it would another block's */
-        auto ownAt = [&](int n) {
-            return S > 1 && n / S == b ? (int)(regions - lds) + r.bytes * (n - b * S) + r.own : -1;
-        };
+        /* (with S = 1 no neighbour is in the block: denseSweepTeam's m > 1) */
+        auto ownAt = [&](int n) { return n / S == b ? (int)(regions - lds) + r.bytes * (n - b * S) + r.own : -1; };
         watcherLoop<real>(a, y, lds, region, r, ownAt(nb.n[0]), ownAt(nb.n[1]));
     } else {
         sweeperLoop<real>(a, y, expTab, hS, region, r);
@@ -755,6 +752,7 @@ void denseSweepTeam(const SweepArgs<real> &args, int slicesPerBlock, size_t maxL
                 "team sweep: bad row of %d sites in %d", args.N, args.Np);
     SQ_THROW_IF(slicesPerBlock < 1 || slicesPerBlock > kTeamMaxSlices, "slices per block out of range (1..%d)",
                 kTeamMaxSlices);
+    SQ_THROW_IF(args.m == 1 && !args.sa, "team sweep: a slice that is its own neighbour");
     SQ_THROW_IF(!args.Qout || args.Qout == args.Qbits, "the sweep needs a second spin buffer");
     SQ_THROW_IF(!args.P || args.ldP < teamWordStride(args.N), "team sweep: no decision words");
     const int nBlocks = divru(args.m, slicesPerBlock);

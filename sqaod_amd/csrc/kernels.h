@@ -157,8 +157,7 @@ struct FieldGemmJob {
  * [blockStart[j], blockStart[j] + fieldGemmJobBlocks(job j)); totalBlocks is the sum.
  * checkFieldGemmJob validates a job's shape on the host. */
 void checkFieldGemmJob(const FieldGemmJob &job, int fieldFormat);
-/* workgroups of a job in a grouped launch (the bf16 forms give a short
- * k-range four column blocks per workgroup) */
+/* workgroups of a job in a grouped launch: a column block by four row tiles each */
 int fieldGemmJobBlocks(const FieldGemmJob &job);
 void fieldRefreshGrouped(int fieldFormat, const FieldGemmJob *d_jobs, const int *d_blockStart, int nJobs,
                          int totalBlocks, hipStream_t stream);
@@ -320,7 +319,8 @@ void launchSweep(void *kernel, int nBlocks, int threads, size_t lds, void **karg
 bool fitsAtOnce(const void *fn, int threads, size_t lds, int nBlocks, int numCUs);
 
 /* The local-field sweep (float: rows of args.J; double) by a team of four waves
- * per slice, each batch ending at its first flip (dense_sweep_team.hip).
+ * per slice, each batch ending at its first flip (dense_sweep_team.hip); not for
+ * one coloring slice, its own neighbour, nor in float at a negative temperature.
  * args.P: m rows of args.ldP >= teamWordStride(N) words; args.tag: 1 to
  * kTeamTagPeriod, no tag twice without P cleared in between. */
 constexpr uint32_t kTeamTagPeriod = 2047;

@@ -590,9 +590,8 @@ def test_more_slices_than_multi_flip_blocks_fit(rocm, N, m, spb, mode):
                                          (100, 2, np.float32), (300, 1, np.float32), (1100, 0, np.float32)])
 def test_one_slice_coloring_bit_exact(oracle, rocm, N, spb, dtype):
     """prepare() selects SA for one slice; the coloring algorithm asked for
-    after it runs with the slice as its own neighbour on both sides.  Alone in
-    its block it keeps no decision words in LDS (spb 0 and 1), with room for
-    another slice it does (2)."""
+    after it runs with the slice as its own neighbour on both sides, by the
+    one-wave kernel."""
     W = dense_int_W(N, SEED_BASE + 13 * N)
     ora, an = make_pair(oracle, rocm, W, 1, seed=17 + N, dtype=dtype, slices_per_block=spb)
     ora.set_algorithm(3)
