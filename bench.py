@@ -412,7 +412,7 @@ def main():
                     help="multi-flip batches of the float local-field forms: auto, on, off or the "
                          "threshold 2..64 (default: the library's, auto)")
     ap.add_argument("--helper-wave", default=None, choices=["on", "off"],
-                    help="second wave per slice applying the deferred rows (default: the library's, on)")
+                    help="a team of four waves per slice (default: the library's, on)")
     ap.add_argument("--no-extras", action="store_true", help="skip the bipartite, BF search and serving runs")
     ap.add_argument("--serve-jobs", type=int, default=48)
     ap.add_argument("--batch-instances", type=int, default=512)

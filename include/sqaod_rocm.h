@@ -89,8 +89,8 @@ int sqaod_rocm_dg_annealer_get_problem_size(sqaod_rocm_dg_annealer *a, int *N);
  * spins were set, when most attempts are accepted, where helper_wave does not
  * apply; the results are the same in every mode),
  * "helper_wave" ("on" | "off": single-flip local-field sweeps run by a team of
- * four waves per slice where they fit in LDS; the results are the same either
- * way),
+ * four waves per slice where all slices' teams fit on the device at once; the
+ * results are the same either way),
  * "slices_per_block" (int, 0 = auto), "sweep_launch" ("auto" | "cooperative"),
  * "refresh_interval" (int, steps between
  * field recomputes; 0 = only after the spins were set), "refresh_engine"

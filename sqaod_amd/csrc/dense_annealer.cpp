@@ -964,10 +964,10 @@ void DenseGraphAnnealer<real>::annealOneStep(real G, real beta) {
         teamS = denseSweepTeamSlices(N_, Np_, m_, sizeof(real), slicesPerBlock_, dev_->numCUs(), dev_->maxLdsPerBlock());
     /* multi-flip batches where LDS allows (float local-field sweeps; the fp8
      * form's on the float copy of J' as well).  "auto" takes them in the first
-     * sweeps only beside the one-wave kernel: the team sweep is faster there but
-     * for the very first sweep of some sizes (us, sweeps 0-2, multi-flip / team:
-     * N=4096, m=256 1980 1260 969 / 1897 1019 677; N=2048, m=128 851 549 428 /
-     * 970 533 350; N=128, m=32 136 109 108 / 71 47 33) */
+     * sweeps only beside the one-wave kernel: the three together are no slower by
+     * the team (us, sweeps 0-2, multi-flip / team: N=4096, m=256 1986 1267 974 /
+     * 1893 1012 660; N=2048, m=128 855 558 432 / 977 526 340; N=1200, m=300 580
+     * 407 335 / 640 377 266; N=128, m=32 136 109 108 / 71 47 33) */
     const bool multi = multiFlipMode_ == kMultiFlipOn || (multiFlipMode_ == kMultiFlipAuto && teamS == 0 &&
                                                           sweepsSinceSpinsSet_ < kMultiFlipAutoSweeps);
     int sweepFormat = fieldFormat_;
