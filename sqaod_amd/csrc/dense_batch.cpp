@@ -317,8 +317,8 @@ void GroupedDenseStepper::run(Device &dev, const std::vector<DenseGraphAnnealer<
             HIP_CHECK(hipStreamEndCapture(st, &g));
             HIP_CHECK(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0));
             HIP_CHECK(hipEventRecord(e0, st));
-            launched = true;
             HIP_CHECK(hipGraphLaunch(ge, st));
+            launched = true;
             HIP_CHECK(hipEventRecord(e1, st));
         } else {
             HIP_CHECK(hipEventRecord(e0, st));
